@@ -199,7 +199,11 @@ class HipForward:
         self._key = None
 
     def _param_key(self, device) -> tuple:
-        return (str(device), self.precision) + tuple(
+        # "cuda" and "cuda:<current>" are one device: keyed apart, a caller that
+        # names it one way and tensors that name it the other would re-pack the
+        # weights at every switch
+        index = torch.cuda.current_device() if device.index is None else device.index
+        return (device.type, index, self.precision) + tuple(
             (p.data_ptr(), p._version) for p in self.net.parameters()
         )
 

@@ -761,3 +761,19 @@ def test_attn_keys_table_matches_restatement():
     for p in range(B):
         bad = np.nonzero(got[p] != want[p])[0]
         assert bad.size == 0, (p, bad[:8], got[p][bad[:8]], want[p][bad[:8]])
+
+
+def test_evaluator_keeps_its_packed_weights():
+    """A device named without an index ("cuda") is the tensors' "cuda:0": a
+    payload of several groups neither packs nor re-packs what the forward
+    already holds."""
+
+    from shrimp import synthetic
+    from shrimp.inference import ShrimpEvaluator
+
+    net = _net(32, 4, "CCA", seed=3)
+    rt = net.hip_runtime()
+    packed = rt.weights(torch.device("cuda:0"))
+    payload, _ = synthetic.serve_payload("cfg4_spec", 10)
+    ShrimpEvaluator(net, "cuda").evaluate_payload(payload)
+    assert rt._packed is packed

@@ -1293,11 +1293,17 @@ static int launch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_b
 // (keys streamed through LDS, one query row per thread).
 static const size_t kAttnSmemCap = 64 * 1024;
 int attn_rows_bf16(const shrimp_attn_args* a, hipStream_t st);
+// Keys streamed through LDS (attn_stream.hip): padded head dims 32 and 64.
+bool attn_stream_ok(const shrimp_attn_args* a, int npos);
+int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
+                       uint32_t o_bytes, hipStream_t st);
 
 template <bool PAIR>
 static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_bytes, int npos,
                          int tab_rows, hipStream_t st) {
   if (g_attn_variant == 3) return attn_rows_bf16(a, st);
+  if (attn_stream_ok(a, npos))
+    return launch_attn_stream(a, qk_scale, qkv_bytes, npos, attn_out_bytes(a), st);
 #define SHRIMP_ATTN_DP(DPV)                                                                \
   if (a->dpad == DPV) {                                                                    \
     const size_t s2 = attn_smem_bytes(DPV, 2, a->S, tab_rows, PAIR);                       \

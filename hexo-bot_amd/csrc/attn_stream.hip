@@ -1,0 +1,616 @@
+// Attention with keys streamed through LDS, for head dims padded to 32 or 64
+// (the 96- and 192-channel networks and the operator ABI's larger heads) at
+// any sequence length. Same semantics as attn.hip: softmax(q k^T / sqrt(d) +
+// bias) v, keys past seq_lens never visited, masked cells weight 0
+// (packages/shrimp/python/shrimp/model.py:448-492, _triton_attn.py:59-130).
+//
+// One workgroup = one (position, head) and 64 QB queries (QB blocks of 16 per
+// wave, four waves). K and V rows arrive 64 keys at a time by buffer-to-LDS
+// DMA, two buffers, the next chunk requested under the current one's products,
+// so LDS does not grow with the sequence beyond 9 bytes per key and three
+// workgroups share a compute unit at D = 64 (the whole-sequence kernel held
+// one, and at S > 560 did not fit at all). Rows lie as in memory (2 D bytes),
+// their 16-byte pieces XOR-swizzled by row so the reads spread over the banks:
+//   K: lane (lr, lg) reads piece 4 ks + lg of key lr = the A operand of a
+//      16x16x32 product, two products per 16 keys x 16 queries at D = 64;
+//   V: ds_read_b64_tr_b16 transposes on the way out: lanes 16 lg .. + 15 address
+//      keys 4 lg .. + 3 (four lanes, 16 dims each) and lane lr receives dim lr
+//      of those four keys, the A operand of V^T P^T.
+// All products stay transposed (S^T = K Q^T, O^T = V^T P^T), so a lane's scores
+// are already its slice of the next product's B operand.
+//
+// Softmax in base 2 around a per-query offset m that moves only when a score
+// exceeds m by more than 2^8 (or no live key was seen yet): the accumulators
+// start at -m / scale, so fma(s, scale, bias) is score - m and the common chunk
+// has no rescale and no lane exchange. Row sums come from a product with ones.
+//
+// Biases, fp32 tables in LDS. LINEAR: the offsets the live cells span, laid out
+// (2 dq_max + 1) x (2 dr_max + 1) without clamping while they fit MAX_OFFSETS
+// (spans of 28 x 28), so a score's bias is one read at kkey[key] - qkey[query];
+// CLAMP: the clamped table of wider positions (13.7 VALU per score against
+// 4.8); PAIR: table rows from the pair tensor. Key blocks that hold token or
+// dead keys, and waves whose queries hold tokens, select per lane.
+//
+// Bound: VALU issue (about 45 instructions per 16 x 32 scores: an address, an
+// fma, an exp, half a maximum and half a pack per score) plus the MFMAs, 66 % of
+// the SIMD cycles together, the rest the chain of one chunk. Measured on MI355X:
+// 111 positions, S = 584, H = 3, D = 64 1873 us (one query row per thread) -> 80 us;
+// 150 positions, S = 328, H = 4, D = 32 67 -> 41 us; the pair tensor at 60
+// positions, S = 341, H = 3, D = 64 94 -> 25.5 us. Two 32-key steps per chunk as a
+// rolled loop keep 139 VGPRs (unrolled 168 with 49 spilled).
+#include <type_traits>
+
+#include "capi.hpp"
+#include "common.hpp"
+
+namespace shrimp {
+
+#define AST_LOG2E 1.4426950408889634f
+#define AST_NEG_BIG (-1.0e30f)
+
+namespace {
+
+enum : int { KEY_CELL = 0, KEY_TOKEN = 1, KEY_DEAD = 2 };
+enum : int { PATH_CLAMP = 0, PATH_LINEAR = 1, PATH_PAIR = 2 };
+
+constexpr int KC = 64;              // keys per chunk
+constexpr int MAX_OFFSETS = 57 * 57;
+constexpr int TU = 16;              // table rows a wave loads together
+constexpr int MAX_LUT_M = 28;       // (2 M + 1)^2 entries fit the same region
+constexpr float LAZY_MAX = 8.0f; // scores above m + this move the offset
+
+typedef __attribute__((address_space(3))) void lds_dst_t;
+typedef __attribute__((address_space(3))) const unsigned char lds_cu8;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+SHRIMP_DEV int clampi(int x, int m) { return min(max(x, -m), m); }
+
+// LDS byte addresses as plain integers (no base pointer added per read).
+SHRIMP_DEV int lds_addr(const void* p) { return (int)(uintptr_t)(lds_cu8*)p; }
+SHRIMP_DEV float lds_f32(int addr) {
+  return *(__attribute__((address_space(3))) const float*)(uintptr_t)(unsigned)addr;
+}
+SHRIMP_DEV u32x4 lds_16(int addr) {
+  return *(__attribute__((address_space(3))) const u32x4*)(uintptr_t)(unsigned)addr;
+}
+SHRIMP_DEV u32x2 lds_tr(int addr) {
+  return __builtin_bit_cast(
+      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(unsigned)addr));
+}
+
+// Swizzle of row r's 16-byte pieces (D / 8 per row): a 128-byte line of LDS
+// holds one row at D = 64 and two at D = 32.
+template <int D>
+SHRIMP_DEV int swz(int r) {
+  return D == 64 ? (r & 7) : ((r >> 1) & 3);
+}
+
+// Per-wave state of its QB query blocks.
+template <int D, int QB>
+struct StreamQuery {
+  u32x4 qf[QB][D / 32];
+  f32x4 o[QB][D / 16];
+  f32x4 l[QB], cinit[QB];  // row sums and -m / scale, four equal elements each
+  float m[QB];
+  int qkey[QB];         // LINEAR: offset code of the query
+  int qq[QB], qr[QB];   // CLAMP: its coordinates
+  bool qtok[QB];
+};
+
+struct StreamLds {
+  const int* kkey;        // LINEAR: LDS address of the key's table row for offset code 0
+  const int2* kqr;        // CLAMP: coordinates
+  const unsigned char* kcls;
+  const float* tab;       // CLAMP and PAIR tables
+  float tokb[3];          // (cell query, token key), (token query, cell key), (token, token)
+  float inv_scale;
+  int npos;
+};
+
+// Key blocks of a chunk scored together: more keep more independent products
+// in flight, fewer fit the registers of three waves per SIMD.
+template <int D, int QB>
+constexpr int stream_nkb() {
+  return QB == 2 ? 2 : 4;
+}
+
+// NKB blocks of 16 keys from key k0, K and V rows at LDS bytes kbuf, vbuf;
+// bit kb of `special` (wave-uniform): block kb selects its biases per lane.
+template <int D, int QB, int PATH, int NKB>
+SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
+                             int k0, int L, int special, int kbuf, int vbuf, int lr, int lg,
+                             float scale, const unsigned (&pd)[QB][NKB]) {
+  constexpr int KS = D / 32, KD = D / 16, RB = 2 * D;
+  f32x4 v[QB][NKB];
+  const int ksw = swz<D>(lr);
+#pragma unroll
+  for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const u32x4 kf = lds_16(kbuf + (kb * 16 + lr) * RB + (((ks * 4 + lg) ^ ksw) << 4));
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+        v[qb][kb] = mfma16x16x32(kf, w.qf[qb][ks], ks == 0 ? w.cinit[qb] : v[qb][kb]);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int kb = 0; kb < NKB; ++kb) {
+    const int key0 = k0 + kb * 16 + lg * 4;
+    int4 kk{0, 0, 0, 0}, kr{0, 0, 0, 0};
+    if constexpr (PATH == PATH_LINEAR) {
+      kk = *reinterpret_cast<const int4*>(s.kkey + key0);
+    } else if constexpr (PATH == PATH_CLAMP) {
+      const int4 a0 = *reinterpret_cast<const int4*>(s.kqr + key0);
+      const int4 a1 = *reinterpret_cast<const int4*>(s.kqr + key0 + 2);
+      kk = int4{a0.x, a0.z, a1.x, a1.z};
+      kr = int4{a0.y, a0.w, a1.y, a1.w};
+    }
+    const int kv[4] = {kk.x, kk.y, kk.z, kk.w}, rv[4] = {kr.x, kr.y, kr.z, kr.w};
+    float bias[QB][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        if constexpr (PATH == PATH_LINEAR) {
+          bias[qb][j] = lds_f32(kv[j] - w.qkey[qb]);
+        } else if constexpr (PATH == PATH_CLAMP) {
+          const int M = a.lut_m, W = 2 * M + 1;
+          bias[qb][j] = s.tab[(clampi(kv[j] - w.qq[qb], M) + M) * W + clampi(rv[j] - w.qr[qb], M) + M];
+        } else {
+          const int p = (int)((pd[qb][kb] >> (8 * j)) & 0xFF);
+          bias[qb][j] = s.tab[min(p, s.npos - 1)];
+        }
+      }
+    if ((special >> kb) & 1) {
+      unsigned cls = 0;
+      if constexpr (PATH != PATH_PAIR) cls = *reinterpret_cast<const unsigned*>(s.kcls + key0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = (cls >> (8 * j)) & 0xFF;
+        const bool dead = PATH == PATH_PAIR ? key0 + j >= L : c == KEY_DEAD;
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+          if constexpr (PATH != PATH_PAIR) {
+            const float ct = w.qtok[qb] ? s.tokb[1] : bias[qb][j];
+            const float tt = w.qtok[qb] ? s.tokb[2] : s.tokb[0];
+            bias[qb][j] = c == KEY_TOKEN ? tt : ct;
+          }
+          // dead keys' K rows are zero, so this is their score: exp2 of it is 0
+          // against any offset (offsets are real scores)
+          if (dead) bias[qb][j] = AST_NEG_BIG;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) v[qb][kb][j] = fmaf(v[qb][kb][j], scale, bias[qb][j]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // does any query's offset have to move?
+  float mx[QB];
+  bool bad = false;
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    float t = v[qb][0][0];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t = fmaxf(t, v[qb][kb][j]);
+    mx[qb] = t;
+    bad |= t > LAZY_MAX || !(w.l[qb][0] > 0.f);
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const float g = max_groups_swap(mx[qb]);
+      const bool seen = w.l[qb][0] > 0.f;
+      // no live key yet: the offset goes to this block's maximum, if it has one
+      const float delta = seen ? fmaxf(g, 0.f) : (g > 0.1f * AST_NEG_BIG ? g : 0.f);
+      const float alpha = seen ? __builtin_amdgcn_exp2f(-delta) : 0.f;
+      w.m[qb] += delta;
+      const float c = -w.m[qb] * s.inv_scale, lsum = w.l[qb][0] * alpha;
+      w.cinit[qb] = f32x4{c, c, c, c};
+      w.l[qb] = f32x4{lsum, lsum, lsum, lsum};
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd) w.o[qb][kd] = w.o[qb][kd] * alpha;
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[qb][kb][j] -= delta;
+    }
+  }
+  u32x2 pf[QB][NKB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+      float p[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(v[qb][kb][j]);
+      pf[qb][kb] = u32x2{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  const unsigned one2 = 0x3F803F80u;
+  const int vrow = 4 * lg + (lr >> 2);
+  const int vsw = swz<D>(vrow);
+  const int vlane = vbuf + vrow * RB + (lr & 1) * 8;
+#pragma unroll
+  for (int kp = 0; kp < NKB; kp += 2) {
+    u32x4 pp[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      pp[qb] = u32x4{pf[qb][kp].x, pf[qb][kp].y, pf[qb][kp + 1].x, pf[qb][kp + 1].y};
+      w.l[qb] = mfma16x16x32(u32x4{one2, one2, one2, one2}, pp[qb], w.l[qb]);
+    }
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) {
+      const int at = vlane + kp * 16 * RB + (((kd * 2 + ((lr & 3) >> 1)) ^ vsw) << 4);
+      const u32x2 v0 = lds_tr(at), v1 = lds_tr(at + 16 * RB);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+        w.o[qb][kd] = mfma16x16x32(u32x4{v0.x, v0.y, v1.x, v1.y}, pp[qb], w.o[qb][kd]);
+    }
+  }
+}
+
+// LDS layout (bytes): [K, V chunk 0][K, V chunk 1][tables][kkey 4 SC or kqr 8 SC]
+// [kcls SC][flags], SC = S rounded up to whole chunks; coords mode only past
+// the tables. 51.6 KB at D = 64 and S = 584: three workgroups per compute unit.
+__host__ __device__ inline int stream_keys(int S) { return (S + KC - 1) / KC * KC; }
+__host__ __device__ inline int stream_tab_bytes(bool pair, int npos) {
+  return pair ? (npos * 4 + 15) / 16 * 16 : (MAX_OFFSETS * 4 + 15) / 16 * 16;
+}
+
+template <int D, int QB, bool PAIR>
+__global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const shrimp_attn_args a, float scale,
+                                                             uint32_t qkv_bytes, int npos,
+                                                             uint32_t o_bytes, int tiles) {
+  constexpr int KS = D / 32, KD = D / 16, RB = 2 * D;
+  constexpr int CB = KC * RB;         // bytes of one chunk's K (or V) rows
+  constexpr int PPR = D / 8;          // 16-byte pieces per row
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ int span_red[4][4];
+
+  // consecutive ids on one XCD (workgroups are dealt to the 8 XCDs round-robin),
+  // so the query tiles of a (position, head) read K and V through one L2
+  const int n = (int)gridDim.x;
+  const int xcd = (int)blockIdx.x & 7, nq = n >> 3, nr = n & 7;
+  const int id = xcd * nq + min(xcd, nr) + ((int)blockIdx.x >> 3);
+  const int bh = id / tiles, tile = id - bh * tiles;
+  const int b = bh / a.H, h = bh - b * a.H;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int lr = lane & 15, lg = lane >> 4;
+  const int S = a.S, SC = stream_keys(S), nt = a.n_tokens, NC = S - nt, H = a.H;
+  int L = a.seq_lens[b];
+  SHRIMP_DCHECK(L >= 0 && L <= S, SHRIMP_DBG_SEQ_LEN);
+  L = L < 0 ? 0 : (L > S ? S : L);
+
+  const __amdgpu_buffer_rsrc_t ors = make_rsrc(a.o, o_bytes);
+  const int qw = tile * (64 * QB) + wave * (16 * QB);  // the wave's first query
+  StreamQuery<D, QB> w;
+  auto store = [&]() {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const int query = qw + qb * 16 + lr;
+      const bool on = query < L;
+      const float inv = on && w.l[qb][0] > 0.f ? 1.0f / w.l[qb][0] : 0.f;
+      const int64_t orow = (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)query * a.o_sr;
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd) {
+        const int e = kd * 16 + lg * 4;
+        u32x2 pk;
+        pk.x = pack_bf16x2(w.o[qb][kd][0] * inv, w.o[qb][kd][1] * inv);
+        pk.y = pack_bf16x2(w.o[qb][kd][2] * inv, w.o[qb][kd][3] * inv);
+        if (!on) pk = u32x2{0u, 0u};
+        __builtin_amdgcn_raw_buffer_store_b64(
+            pk, ors, query < S && e < a.d ? (uint32_t)((orow + e) * 2) : SHRIMP_OOB_OFFSET, 0, 0);
+      }
+    }
+  };
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    w.m[qb] = 0.f;
+    w.l[qb] = w.cinit[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    w.qkey[qb] = w.qq[qb] = w.qr[qb] = 0;
+    w.qtok[qb] = qw + qb * 16 + lr < nt;
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) w.o[qb][kd] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (tile * (64 * QB) >= L) {  // uniform: only rows past the bound
+    store();
+    return;
+  }
+
+  unsigned char* tabs = smem + 4 * CB;
+  int2* kqr = reinterpret_cast<int2*>(tabs + stream_tab_bytes(PAIR, npos));
+  int* kkey = reinterpret_cast<int*>(kqr);
+  unsigned char* kcls = reinterpret_cast<unsigned char*>(kqr + SC);
+  unsigned char* flags = kcls + SC;  // per chunk: bit kb, key block kb holds a token or dead key
+
+  const int64_t base = (int64_t)b * a.qkv_sb + (int64_t)h * a.qkv_sh;
+  const __amdgpu_buffer_rsrc_t qrs = make_rsrc(a.q, qkv_bytes);
+  const __amdgpu_buffer_rsrc_t krs = make_rsrc(a.k, qkv_bytes);
+  const __amdgpu_buffer_rsrc_t vrs = make_rsrc(a.v, qkv_bytes);
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int query = qw + qb * 16 + lr;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      w.qf[qb][ks] = buf_load16(
+          qrs, query < L ? (uint32_t)((base + query * D + ks * 32 + lg * 8) * 2) : SHRIMP_OOB_OFFSET);
+  }
+
+  // 1 KiB DMAs of a chunk's K, then V rows: lane -> (row, slot), the slot's
+  // piece by the row's swizzle; dead keys land as zeros
+  auto dma = [&](int c, int buf) {
+#pragma unroll
+    for (int i = 0; i < 2 * PPR / 4; ++i) {
+      const int j = wave + 4 * i;
+      const int tensor = j >= PPR ? 1 : 0;
+      const int row = (j - tensor * PPR) * (64 / PPR) + lane / PPR;
+      const int piece = (lane % PPR) ^ swz<D>(row);
+      const int key = c * KC + row;
+      const bool ok = PAIR ? key < L : kcls[key] != KEY_DEAD;
+      const uint32_t off =
+          ok ? (uint32_t)((base + (int64_t)key * D + piece * 8) * 2) : SHRIMP_OOB_OFFSET;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(tensor ? vrs : krs,
+                                               (lds_dst_t*)(smem + buf * 2 * CB + j * 1024), 16, off,
+                                               0, 0, 0);
+    }
+  };
+  StreamLds s;
+  s.kkey = kkey;
+  s.kqr = kqr;
+  s.kcls = kcls;
+  s.tab = reinterpret_cast<const float*>(tabs);
+  s.npos = npos;
+  s.inv_scale = 1.0f / scale;
+  bool linear = false;
+  if constexpr (PAIR) {
+    for (int i = tid; i < npos; i += 256)
+      reinterpret_cast<float*>(tabs)[i] = a.table2[(int64_t)i * H + h] * AST_LOG2E;
+  } else {
+    // key classes and coordinates, span of the live cells
+    int qmin = 1 << 30, qmax = -(1 << 30), rmin = 1 << 30, rmax = -(1 << 30);
+    for (int key = tid; key < SC; key += 256) {
+      int q = 0, r = 0, cls = KEY_DEAD;  // keys past the bound (tokens too) are dead
+      if (key < nt && key < L) {
+        cls = KEY_TOKEN;
+      } else if (key >= nt && key < L) {
+        const int64_t cell = (int64_t)b * NC + (key - nt);
+        q = a.coords[cell * 2];
+        r = a.coords[cell * 2 + 1];
+        cls = a.mask[cell] != 0 ? KEY_CELL : KEY_DEAD;
+        if (cls == KEY_CELL) {
+          qmin = min(qmin, q);
+          qmax = max(qmax, q);
+          rmin = min(rmin, r);
+          rmax = max(rmax, r);
+        }
+      }
+      kcls[key] = (unsigned char)cls;
+      // a wave covers one whole chunk per iteration
+      const uint64_t sp = __builtin_amdgcn_ballot_w64(cls != KEY_CELL);
+      if (lane == 0)
+        flags[key / KC] = (unsigned char)(((sp & 0xFFFFu) != 0) | ((sp >> 16 & 0xFFFFu) != 0) << 1 |
+                                          ((sp >> 32 & 0xFFFFu) != 0) << 2 | ((sp >> 48) != 0) << 3);
+    }
+    for (int m = 32; m >= 1; m >>= 1) {
+      qmin = min(qmin, __shfl_xor(qmin, m, 64));
+      qmax = max(qmax, __shfl_xor(qmax, m, 64));
+      rmin = min(rmin, __shfl_xor(rmin, m, 64));
+      rmax = max(rmax, __shfl_xor(rmax, m, 64));
+    }
+    if (lane == 0) {
+      span_red[wave][0] = qmin;
+      span_red[wave][1] = qmax;
+      span_red[wave][2] = rmin;
+      span_red[wave][3] = rmax;
+    }
+    const int W2 = (2 * a.lut_m + 1) * (2 * a.lut_m + 1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.tokb[i] = a.btab[(int64_t)(W2 + i) * H + h];
+    __syncthreads();
+    dma(0, 0);  // under the table's round trip
+    int q0 = span_red[0][0], q1 = span_red[0][1], r0 = span_red[0][2], r1 = span_red[0][3];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+      q0 = min(q0, span_red[i][0]);
+      q1 = max(q1, span_red[i][1]);
+      r0 = min(r0, span_red[i][2]);
+      r1 = max(r1, span_red[i][3]);
+    }
+    // LINEAR needs a live cell (token and dead keys borrow its code) and the
+    // spanned offsets to fit the table region
+    const int64_t sq = (int64_t)q1 - q0, sr = (int64_t)r1 - r0;
+    linear = sq >= 0 && sq < MAX_OFFSETS && sr < MAX_OFFSETS &&
+             (2 * sq + 1) * (2 * sr + 1) <= MAX_OFFSETS;
+    const int M = a.lut_m, W = 2 * M + 1, XW = linear ? 2 * (int)sr + 1 : 0;
+    float* tab = reinterpret_cast<float*>(tabs);
+    if (linear) {
+      // a wave per row of offsets dq, lanes along dr; a thread's loads all issued
+      // before its stores (one by one they cost 14 round trips, 5 us per workgroup)
+      for (int c0 = 0; c0 < XW; c0 += 64) {
+        const int dr = c0 + lane;
+        const int col = (clampi(dr - (int)sr, M) + M) * H + h;
+        for (int d0 = wave; d0 <= 2 * (int)sq; d0 += 4 * TU) {
+          float t[TU];
+#pragma unroll
+          for (int u = 0; u < TU; ++u) {
+            const int dq = min(d0 + 4 * u, 2 * (int)sq);
+            t[u] = a.btab[(int64_t)(clampi(dq - (int)sq, M) + M) * W * H + col];
+          }
+#pragma unroll
+          for (int u = 0; u < TU; ++u)
+            if (dr < XW && d0 + 4 * u <= 2 * (int)sq) tab[(d0 + 4 * u) * XW + dr] = t[u];
+        }
+      }
+    } else {
+      for (int i = tid; i < W2; i += 256) tab[i] = a.btab[(int64_t)i * H + h];
+    }
+    // LINEAR: token and dead keys take the code of the live cell (q0, r0), so
+    // every read stays inside the table; their biases are selected afterwards
+    const int xoff = lds_addr(tabs) + (linear ? ((int)sq * XW + (int)sr) * 4 : 0);
+    auto code = [&](int2 c) { return ((c.x - q0) * XW + (c.y - r0)) * 4; };
+    auto cell_of = [&](int key) {
+      const int64_t cell = (int64_t)b * NC + (key - nt);
+      return make_int2(a.coords[cell * 2], a.coords[cell * 2 + 1]);
+    };
+    for (int key = tid; key < SC; key += 256) {
+      const bool cell = kcls[key] == KEY_CELL;
+      if (linear) kkey[key] = xoff + (cell ? code(cell_of(key)) : 0);
+      else kqr[key] = cell ? cell_of(key) : make_int2(0, 0);
+    }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const int query = qw + qb * 16 + lr;
+      w.qq[qb] = w.qr[qb] = w.qkey[qb] = 0;
+      if (query < L && kcls[query] == KEY_CELL) {
+        const int2 c = cell_of(query);
+        w.qq[qb] = c.x;
+        w.qr[qb] = c.y;
+        if (linear) w.qkey[qb] = code(c);
+      }
+    }
+  }
+
+  // pair rows of a chunk: four table rows per 16-key block and lane
+  unsigned pn[QB][4];
+  auto load_pair = [&](int c, unsigned (&p)[QB][4]) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const int query = qw + qb * 16 + lr;
+      const uint8_t* row = a.pair + (int64_t)b * a.p_sb + (int64_t)(query < L ? query : 0) * a.p_sq;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const int key = c * KC + kb * 16 + lg * 4;
+        unsigned x = 0;
+        if (c * KC + KC <= S) {
+          __builtin_memcpy(&x, row + key, 4);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (key + j < S) x |= (unsigned)row[key + j] << (8 * j);
+        }
+        p[qb][kb] = x;
+      }
+    }
+  };
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) pn[qb][kb] = 0;
+
+  const int nc = (L + KC - 1) / KC;
+  const bool active = qw < L;
+  const bool tok = !PAIR && qw < nt;  // the wave's queries hold tokens
+  const int lds0 = lds_addr(smem);
+  if (PAIR) dma(0, 0);
+  if (PAIR && active) load_pair(0, pn);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  // one loop per bias path: the paths share no registers
+  auto run = [&](auto path) {
+    for (int c = 0; c < nc; ++c) {
+      const int buf = c & 1;
+      unsigned pd[QB][4];
+      if constexpr (PAIR) {
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) pd[qb][kb] = pn[qb][kb];
+      }
+      if (c + 1 < nc) {
+        dma(c + 1, buf ^ 1);
+        if (PAIR && active) load_pair(c + 1, pn);
+      }
+      if (active) {
+        const int kbuf = lds0 + buf * 2 * CB, vbuf = kbuf + CB;
+        constexpr int NKB = stream_nkb<D, QB>();
+        int special;
+        if constexpr (PAIR) {
+          const int over = L - c * KC;  // keys of the chunk inside the bound
+          special = over >= KC ? 0 : (15 << (over >> 4)) & 15;
+        } else {
+          special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)flags[c]);
+        }
+#pragma unroll 1
+        for (int kb = 0; kb < 4 && c * KC + kb * 16 < L; kb += NKB) {
+          unsigned p[QB][NKB];
+          if constexpr (PAIR) {
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+              for (int i = 0; i < NKB; ++i) p[qb][i] = kb == 0 ? pd[qb][i] : pd[qb][(4 - NKB) + i];
+          }
+          stream_chunk<D, QB, decltype(path)::value, NKB>(
+              a, w, s, c * KC + kb * 16, L, special >> kb, kbuf + kb * 16 * RB, vbuf + kb * 16 * RB,
+              lr, lg, scale, p);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
+  };
+  if constexpr (PAIR) {
+    run(std::integral_constant<int, PATH_PAIR>{});
+  } else {
+    if (linear) run(std::integral_constant<int, PATH_LINEAR>{});
+    else run(std::integral_constant<int, PATH_CLAMP>{});
+  }
+  store();
+}
+
+size_t stream_smem(int D, bool pair, int S, int npos) {
+  const size_t SC = (size_t)stream_keys(S);
+  return (size_t)4 * KC * 2 * D + stream_tab_bytes(pair, npos) +
+         (pair ? 0 : SC * 9 + (SC / KC + 15) / 16 * 16);
+}
+
+}  // namespace
+
+// Whether the streamed kernel covers the call: padded head dim 32 or 64, q / k
+// / v rows on 16-byte boundaries (DMA pieces), tables within a workgroup's LDS.
+bool attn_stream_ok(const shrimp_attn_args* a, int npos) {
+  if (a->dpad != 32 && a->dpad != 64) return false;
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a->q) | reinterpret_cast<uintptr_t>(a->k) |
+                      reinterpret_cast<uintptr_t>(a->v);
+  if ((p & 15) != 0 || a->qkv_sb % 8 != 0 || a->qkv_sh % 8 != 0) return false;
+  if (a->pair == nullptr && a->lut_m > MAX_LUT_M) return false;
+  if ((int64_t)a->B * a->H * ((a->S + 63) / 64) >= (1 << 30)) return false;
+  return stream_smem(a->dpad, a->pair != nullptr, a->S, npos) <= (size_t)max_lds_per_block();
+}
+
+template <int D, int QB, bool PAIR>
+static int launch_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
+                         uint32_t o_bytes, hipStream_t st) {
+  const int tiles = (a->S + 64 * QB - 1) / (64 * QB);
+  hipLaunchKernelGGL((attn_stream_kernel<D, QB, PAIR>), dim3(a->B * a->H * tiles), dim3(256),
+                     stream_smem(D, PAIR, a->S, npos), st, *a, scale, qkv_bytes, npos, o_bytes, tiles);
+  return check_launch("attn");
+}
+
+// 32 queries per wave (each K and V fragment read feeds two products) once
+// such tiles give every compute unit two workgroups, else 16.
+int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
+                       uint32_t o_bytes, hipStream_t st) {
+  const bool wide = (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
+  const bool pair = a->pair != nullptr;
+#define AST_LAUNCH(DV)                                                                            \
+  if (pair)                                                                                       \
+    return wide ? launch_stream<DV, 2, true>(a, scale, qkv_bytes, npos, o_bytes, st)              \
+                : launch_stream<DV, 1, true>(a, scale, qkv_bytes, npos, o_bytes, st);             \
+  return wide ? launch_stream<DV, 2, false>(a, scale, qkv_bytes, npos, o_bytes, st)               \
+              : launch_stream<DV, 1, false>(a, scale, qkv_bytes, npos, o_bytes, st)
+  if (a->dpad == 64) {
+    AST_LAUNCH(64);
+  }
+  AST_LAUNCH(32);
+#undef AST_LAUNCH
+}
+
+}  // namespace shrimp

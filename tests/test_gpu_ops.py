@@ -1248,3 +1248,67 @@ def test_attn_keys_tokens_equals_separate_launches():
                                        tok.data_ptr(), 16, seq.data_ptr(), 16, None,
                                        _lib.stream_handle()) == -1
     assert "position stride" in lib.shrimp_last_error().decode()
+
+
+def _coords_attention_ref(q, k, v, coords, mask, lens, table, nt):
+    """float64 softmax(q k^T / sqrt(d) + table[pair]) v over live keys below
+    lens; nt token rows (0 or 8) ahead of the cells; rows past lens are 0."""
+
+    B, H, S, d = q.shape
+    pair = torch.from_numpy(tables.pair_rows(coords.numpy(), mask.numpy()))[:, 8 - nt:, 8 - nt:]
+    bias = table.double()[pair].permute(0, 3, 1, 2)
+    below = torch.arange(S)[None, :] < lens[:, None].long()
+    live = torch.cat([torch.ones(B, nt, dtype=torch.bool), mask.bool()], dim=1) & below
+    sc = (q @ k.transpose(-2, -1)) / math.sqrt(d) + bias
+    sc = sc.masked_fill(~live[:, None, None, :], float("-inf"))
+    p = torch.softmax(sc, dim=-1).nan_to_num(0.0)  # a row with no live key gives 0
+    return torch.where(below[:, None, :, None], p @ v, torch.zeros_like(q))
+
+
+# head dims 32 and 64 stream the keys through LDS 64 at a time: sequence
+# lengths around a chunk and around the two query tilings (64 queries per
+# workgroup, or 128 once B H tiles reach two per compute unit: B = 96, H = 6),
+# spans on either side of the unclamped table (window 20: linear, 60: clamped),
+# lengths of 0, inside the tokens and ragged, dead cells whose K and V rows hold
+# NaN, a head dim below its padding, an odd head count
+@pytest.mark.parametrize("gain", [1.0, 20.0])
+@pytest.mark.parametrize("B,H,S,d,dpad,nt,window", [
+    (5, 3, 64, 64, 64, 8, 20), (5, 3, 65, 64, 64, 8, 60), (5, 4, 130, 24, 32, 8, 20),
+    (5, 4, 63, 32, 32, 0, 60), (96, 6, 72, 32, 32, 8, 20), (96, 6, 129, 64, 64, 0, 60),
+    (5, 3, 584, 64, 64, 8, 40),
+])
+def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
+    from shrimp import ops
+    from shrimp.geometry import CELL_LUT_M, cell_bias_lut
+
+    rng = np.random.default_rng(5)
+    N = S - nt
+    cells = np.stack([rng.permutation(window * window)[:N] for _ in range(B)])
+    coords = torch.from_numpy(np.stack([cells // window, cells % window], -1).astype(np.int32)) - 7
+    mask = torch.from_numpy(rng.random((B, N)) < 0.93)
+    lens = torch.from_numpy(rng.integers(nt + 1, S + 1, size=B).astype(np.int32))
+    lens[0], lens[1], lens[2] = S, 0, max(nt // 2, 1)
+    table = torch.from_numpy(rng.standard_normal((237, H)).astype(np.float32))
+    q, k, v = (torch.from_numpy(rng.standard_normal((B, H, S, d)).astype(np.float32)) for _ in range(3))
+    qb, kb, vb = bf(q * gain), bf(k), bf(v)
+    want = _coords_attention_ref(qb, kb, vb, coords, mask, lens, table, nt)
+    dead = torch.cat([torch.zeros(B, nt, dtype=torch.bool), ~mask], dim=1)
+
+    def dev(t, nan):
+        t = torch.nn.functional.pad(t, (0, dpad - d)).to(torch.bfloat16)
+        return torch.where(dead[:, None, :, None] & nan, float("nan"), t).to(DEV).contiguous()
+
+    btab, xtab = ops.attn_bias_table(table.to(DEV), torch.from_numpy(cell_bias_lut()).to(DEV))
+    out = torch.full((B, H, S, d), 7.0, dtype=torch.bfloat16, device=DEV)
+    # the caller's buffers stay referenced until the launch is done
+    qd, kd, vd = dev(qb, False), dev(kb, True), dev(vb, True)
+    cd, md, ld = coords.to(DEV), mask.to(DEV, torch.uint8), lens.to(DEV)
+    ops.launch_attn(q=qd, k=kd, v=vd, qkv_sb=H * S * dpad, qkv_sh=S * dpad, seq_lens=ld, o=out,
+                    o_sb=H * S * d, o_sh=S * d, o_sr=d, B=B, S=S, H=H, d=d, dpad=dpad, coords=cd,
+                    mask8=md, btab=btab, xtab=xtab, lut_m=CELL_LUT_M, n_tokens=nt)
+    # a dead query row is not specified beyond being finite (the callers mask it)
+    rows = ~dead[:, None, :, None].expand_as(want)
+    got = out.cpu().double()
+    assert torch.isfinite(got).all()
+    # p and the result are rounded to bf16 (2^-9 each) around |v| up to 4.5
+    close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")

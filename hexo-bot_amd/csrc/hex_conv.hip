@@ -146,6 +146,8 @@ SHRIMP_DEV void conv_epilogue(const shrimp_conv_args& a, f32x4 (&acc)[COUT / 16]
 
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
+    // (192 channels: keep the parameters of one block from being held for the next)
+    if constexpr (NB > 8) asm volatile("" ::: "memory");
     float v[NB][4];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -681,6 +683,165 @@ __global__ __launch_bounds__(256, 2) void hex_conv_lds_kernel(const shrimp_conv_
     }
     lds_conv_epilogue<COUT, MB, EPI, B16>(a, acc, rb, rn, rv, lg, lp, o_bytes, r_bytes);
   }
+}
+
+// Weight-streamed variant (7 taps, widths without a big-tile instance: 96 and
+// 192 channels, and their 32-channel stems): a workgroup owns 64 MB rows of the
+// flattened (position, cell) rows, MB blocks of 16 per wave and all COUT
+// channels, for any N. Rows are gathered straight into MFMA fragments (L2, two
+// steps ahead); each weight fragment comes from L2 once per workgroup, by DMA
+// into a ring of three LDS stages two stages ahead, and feeds the four waves:
+// the global-gather kernel read the whole weight (516 KB at 192 channels) once
+// per wave, 1 GB through the L2 per launch, and was bound by that (63 936 rows at
+// 192 channels, LN + ReLU: 69 -> 42.2 us, 782 TFLOP/s; 48 000 rows at 96
+// channels: 24.8 -> 16.6 us). Now bound by the MFMAs at 192 channels and, at 96
+// and for small batches, by the stage chain of one workgroup. The K order
+// (tap outer, channel chunk inner) and the epilogue arithmetic are the
+// global-gather kernel's, so MB does not change the bits.
+//
+// Requests retire in order (vmcnt), so at the top of stage g the DMAs of stage
+// g, issued at the top of g - 2, are complete once at most the requests issued
+// during g - 1 are outstanding: WAIT counts the fewest of those. The barrier
+// then makes every wave's part visible and frees the slot that stage g - 1 read.
+// LDS reads go through integer addresses: through a pointer the compiler takes
+// them to alias the DMAs in flight and waits for all of them.
+typedef __attribute__((address_space(3))) void ws_lds_t;
+SHRIMP_DEV u32x4 ws_lds16(int addr) {
+  return *(__attribute__((address_space(3))) const u32x4*)(uintptr_t)(unsigned)addr;
+}
+
+constexpr int ws_sps(int kc) { return kc == 6 ? 2 : kc; }  // K steps per stage
+constexpr size_t ws_lds_bytes(int cout, int cin) {
+  return (size_t)3 * ws_sps(cin / 32) * (cout / 16) * 1024 + (size_t)5 * cout * 4;
+}
+
+template <int COUT, int CIN, int MB, int EPI>
+__global__ __launch_bounds__(256, 2) void hex_conv_ws_kernel(
+    const shrimp_conv_args a, uint32_t x_bytes, uint32_t w_bytes, uint32_t o_bytes,
+    uint32_t r_bytes) {
+  constexpr int NB = COUT / 16, KC = CIN / 32, T = 7;
+  constexpr int SPS = ws_sps(KC), SPT = KC / SPS;   // steps per stage, stages per tap
+  constexpr int SF = SPS * NB;                      // fragments (1 KiB) per stage
+  constexpr int DMIN = SF / 4;                      // fewest DMAs of a wave per stage
+  constexpr int NSTAGE = T * SPT;
+  constexpr int PD = KC == 1 ? 1 : 2;               // row prefetch distance (steps)
+  constexpr int WAIT = DMIN + SPS * MB;
+  static_assert(KC % SPS == 0 && WAIT < 64, "whole stages per tap; vmcnt is 6 bits");
+  extern __shared__ __attribute__((aligned(16))) unsigned char xs[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int lr = lane & 15;
+  const int lg = lane >> 4;
+  const int N = a.N;
+  const int total = a.B * N;
+  // consecutive row tiles on one XCD (workgroups are dealt to the 8 XCDs
+  // round-robin), so a position's rows are gathered through one L2
+  const int nwg = (int)gridDim.x, xcd = (int)blockIdx.x & 7;
+  const int id = xcd * (nwg >> 3) + min(xcd, nwg & 7) + ((int)blockIdx.x >> 3);
+  const int row_base = (id * 4 + wave) * (MB * 16);
+
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, x_bytes);
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.w, w_bytes);
+
+  int rb[MB], rn[MB];
+  bool rv[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int r = row_base + mb * 16 + lr;
+    rv[mb] = r < total;
+    rb[mb] = rv[mb] ? r / N : 0;
+    rn[mb] = rv[mb] ? r - rb[mb] * N : 0;
+  }
+  auto load_idx = [&](int t, int (&j)[MB]) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      j[mb] = -1;
+      if (t < T && rv[mb]) j[mb] = a.idx[(int64_t)(rb[mb] * N + rn[mb]) * a.idx_stride + t];
+    }
+  };
+  // byte offset (this lane's k-slice included) of the gathered rows
+  auto offsets = [&](const int (&j)[MB], uint32_t (&off)[MB]) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      SHRIMP_DCHECK(j[mb] >= -1, SHRIMP_DBG_CONV_INDEX);
+      const bool ok = j[mb] >= 0 && j[mb] < N;
+      const int64_t e = (int64_t)rb[mb] * a.x_sb + (int64_t)j[mb] * a.x_sn;
+      off[mb] = ok ? (uint32_t)(e * 2) + (uint32_t)(lg * 16) : SHRIMP_OOB_OFFSET;
+    }
+  };
+  const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)xs;
+  auto dma = [&](int g, int slot) {  // past the last stage: past the resource, zeros
+#pragma unroll
+    for (int i = 0; i < (SF + 3) / 4; ++i) {
+      const int f = wave + 4 * i;
+      if (SF % 4 == 0 || f < SF)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            wr, (ws_lds_t*)(xs + (slot * SF + f) * 1024), 16,
+            g < NSTAGE ? (uint32_t)((g * SF + f) * 1024 + lane * 16) : SHRIMP_OOB_OFFSET, 0, 0, 0);
+    }
+  };
+
+  float* lp = reinterpret_cast<float*>(xs + 3 * SF * 1024);
+  stage_params<COUT>(lp, a, (EPI & EPI_HEAD) != 0);
+  int jn[MB];
+  uint32_t off[MB], offn[MB];
+  load_idx(0, jn);
+  dma(0, 0);
+  dma(1, 1);
+  offsets(jn, off);
+  load_idx(1, jn);
+  u32x4 xf[PD + 1][MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) xf[0][mb] = buf_load16(xr, off[mb]);
+  if constexpr (PD == 2) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) xf[1][mb] = buf_load16(xr, off[mb] + 64);
+  }
+
+  f32x4 acc[NB][MB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  int slot = 0;  // g % 3
+#pragma unroll(KC == 1 ? T : 1)
+  for (int t = 0; t < T; ++t) {
+    offsets(jn, offn);  // tap t + 1 (none past the last: absent rows)
+    load_idx(t + 2, jn);
+#pragma unroll
+    for (int i = 0; i < SPT; ++i) {
+      const int g = t * SPT + i;
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) __builtin_amdgcn_s_waitcnt(0);
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | (WAIT & 15) | ((WAIT >> 4) << 14));
+      __syncthreads();
+      dma(g + 2, slot == 0 ? 2 : slot - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const int wbase = lds0 + slot * SF * 1024 + lane * 16;
+#pragma unroll
+      for (int s = 0; s < SPS; ++s) {
+        const int k = i * SPS + s;                       // channel chunk of this step
+        const int cur = (KC == 1 ? t : k) % (PD + 1);    // ring slot of its rows
+        const int pk = k + PD, nxt = (KC == 1 ? t + PD : pk) % (PD + 1);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          xf[nxt][mb] = buf_load16(xr, pk < KC ? off[mb] + (uint32_t)(pk * 64)
+                                               : offn[mb] + (uint32_t)((pk - KC) * 64));
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const u32x4 w = ws_lds16(wbase + (s * NB + nb) * 1024);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = mfma16x16x32(w, xf[cur][mb], acc[nb][mb]);
+        }
+      }
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) off[mb] = offn[mb];
+  }
+  lds_conv_epilogue<COUT, MB, EPI, true>(a, acc, rb, rn, rv, lg, lp, o_bytes, r_bytes);
 }
 
 // Big-tile variant for the trunk shape (cin_pad = cout = 128, 7 taps, N <= 512):
@@ -1415,7 +1576,35 @@ static int launch_conv(const shrimp_conv_args* a, uint32_t xb, uint32_t wb, size
   const bool b16 = COUT == 128 && !head && out16 && o_ext < (int64_t)0x7FFF0000 &&
                    r_ext < (int64_t)0x7FFF0000 &&
                    (!(EPI & EPI_RESID) || (a->r_sn % 4 == 0 && a->r_sb % 4 == 0));
+  const bool b16_any = o_ext < (int64_t)0x7FFF0000 && r_ext < (int64_t)0x7FFF0000 &&
+                       (!(EPI & EPI_RESID) || (a->r_sn % 4 == 0 && a->r_sb % 4 == 0));
   const uint32_t ob = (uint32_t)o_ext, rbb = (uint32_t)r_ext;
+  // Weight-streamed kernel. 32 rows per wave (each weight fragment read from LDS
+  // feeds two products) once that gives every compute unit a workgroup, else 16.
+  // Measured (LN + ReLU): 63 936 rows at 192 channels 42.8 us with 32 rows, 52.6
+  // with 16, 48.3 with 64 (one wave per SIMD: nothing under the epilogue);
+  // 29 790 rows 30.3 / 28.5 / 45.2; 48 000 rows at 96 channels 16.3 / 19.6 / 18.8.
+  // The global-gather kernel took 69, 39.6 and 24.8 us.
+  if constexpr (COUT == 96 || COUT == 192) {
+    if ((a->cin_pad == COUT || a->cin_pad == 32) && a->taps == 7 && out16 && b16_any &&
+        (g_conv_variant == 0 || g_conv_variant == 3)) {
+      const int64_t rows = (int64_t)a->B * a->N;
+      const int mb = rows >= (int64_t)128 * cu_count() ? 2 : 1;
+      const dim3 grid((unsigned)((rows + 64 * mb - 1) / (64 * mb)));
+#define SHRIMP_WS(CINV, MBV)                                                                \
+  hipLaunchKernelGGL((hex_conv_ws_kernel<COUT, CINV, MBV, EPI>), grid, dim3(256),            \
+                     ws_lds_bytes(COUT, CINV), st, *a, xb, wb, ob, rbb)
+      if (a->cin_pad == 32) {
+        if (mb == 2) SHRIMP_WS(32, 2);
+        else SHRIMP_WS(32, 1);
+      } else {
+        if (mb == 2) SHRIMP_WS(COUT, 2);
+        else SHRIMP_WS(COUT, 1);
+      }
+#undef SHRIMP_WS
+      return check_launch("hex_conv");
+    }
+  }
 #define SHRIMP_LDS_LAUNCH(GRID, MBV, CINV, BIGO)                                                     \
   do {                                                                                             \
     if (b16)                                                                                       \

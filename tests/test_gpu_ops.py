@@ -1312,3 +1312,53 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     assert torch.isfinite(got).all()
     # p and the result are rounded to bf16 (2^-9 each) around |v| up to 4.5
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
+
+
+# the weight-streamed conv (96 and 192 channels, their 32-channel stems): a last
+# tile of one row, a wave with no rows, and both row tilings (16 rows per wave
+# below 128 rows per compute unit, 32 from there); the K order and epilogue
+# arithmetic are the global-gather kernel's, so the bits are too
+@pytest.mark.parametrize("B,N", [(1, 1), (3, 43), (2, 160), (131, 257)])
+@pytest.mark.parametrize("cin,c", [(96, 96), (192, 192), (15, 96), (15, 192)])
+def test_conv_weight_streamed(cin, c, B, N):
+    from shrimp import _lib, ops
+
+    g = torch.Generator().manual_seed(B * N + c + cin)
+    cp = -(-cin // 32) * 32
+    x = torch.zeros(B, N, cp)
+    x[..., :cin] = torch.randn(B, N, cin, generator=g)
+    mask = torch.rand(B, N, generator=g) < 0.9
+    # any row of the position, absent as N or -1
+    idx = torch.randint(-1, N + 1, (B, N, 7), generator=g, dtype=torch.int32).to(DEV)
+    w = torch.randn(7, cin, c, generator=g) / math.sqrt(7 * cin)
+    par = [torch.randn(c, generator=g).to(DEV) for _ in range(5)]
+    xd, m8 = x.to(DEV, torch.bfloat16), mask.to(DEV, torch.uint8)
+    wp = ops.pack_conv_weight(w.to(DEV), cp)
+    resid = torch.randn(B, N, c, generator=g).to(DEV, torch.bfloat16)
+    hb = torch.randn(1, generator=g).to(DEV)
+    common = dict(x=xd, x_sb=N * cp, x_sn=cp, idx=idx, taps=7, idx_stride=7, mask8=m8, wpack=wp,
+                  bias=par[0], B=B, N=N, cin_pad=cp, cout=c)
+    lib = _lib.load()
+
+    def run(variant):
+        prev = lib.shrimp_conv_variant(variant)
+        outs = []
+        try:
+            ln = dict(ln_w=par[1], ln_b=par[2])
+            for kw in (dict(), dict(relu=True), ln, dict(ln, relu=True),
+                       dict(ln, resid=resid, r_sb=N * c, r_sn=c, gamma=par[3])):
+                out = torch.full((B, N, c), 7.0, dtype=torch.bfloat16, device=DEV)
+                ops.launch_conv(out=out, o_sb=N * c, o_sn=c, **kw, **common)
+                outs.append(out)
+            head = torch.full((B, N), 7.0, device=DEV)
+            ops.launch_conv(relu=True, head_w=par[4], head_b=hb, head_out=head, **common)
+        finally:
+            lib.shrimp_conv_variant(prev)
+        return [*outs, head]
+
+    want = ofwd.hex_conv_ln(bf(x[..., :cin]), idx.cpu(), mask, bf(w), par[0].cpu().double(),
+                            par[1].cpu().double(), par[2].cpu().double(), 1e-5, True)
+    got = run(0)
+    close(got[3], want, what="LN + ReLU")
+    for k, (a, b) in enumerate(zip(got, run(1))):
+        assert torch.equal(a, b), k

@@ -46,6 +46,13 @@ __global__ void pack_weight_kernel(const float* __restrict__ src, unsigned short
                                    int K, int NOUT, int cin, int cin_pad, int64_t s_t,
                                    int64_t s_c, int64_t s_n, int interleaved);
 
+// 96 and 192 channels (block_stream.hip).
+bool block_stream_width(int C);
+size_t mlp_stream_pack_bytes(int C);
+int pack_mlp_stream(const shrimp_mlp_weights* w, unsigned char* pk, float* tmp, hipStream_t st);
+int launch_mlp_stream(const shrimp_mlp_args* a, uint32_t x_bytes, uint32_t s_bytes, uint32_t lo_bytes,
+                      hipStream_t st);
+
 namespace {
 
 constexpr int MC = 128;           // channels
@@ -59,31 +66,6 @@ constexpr uint32_t BO_OFF = W_LDS;                    // folded biases (fp32) af
 constexpr uint32_t B1_OFF = BO_OFF + MC * 4;
 constexpr uint32_t B2_OFF = B1_OFF + MH * 4;
 constexpr uint32_t PACK_BYTES = B2_OFF + MC * 4;
-
-// GELU(x) = x Phi(x) = max(x, 0) - |x| h(|x|), h(a) = erfc(a / sqrt(2)) / 2.
-// h is evaluated as exp2(-g(a)) with g a degree-5 polynomial fitted (weighted
-// least squares on a in [0, 5], weight a h(a)) to -log2 h(a), and a clamped at
-// 5 (h(5) = 2.9e-7): one transcendental and seven fused multiply-adds per
-// value. Against float64 erf-GELU the error is at most 3.8e-6 absolute over
-// [-12, 12] (a tenth of a bf16 rounding step of the output near 0.1), and the
-// kernel rounds the result to bf16 for fc2. The clamp is one med3 and max(x, 0)
-// one integer max (relu_bits): fminf / fmaxf on an MFMA result cost a second
-// instruction each, a canonicalisation of the operand the compiler cannot
-// prove canonical.
-SHRIMP_DEV float gelu_ex2(float x) {
-  constexpr float g0 = 1.0001733303070068f, g1 = 1.149885654449463f, g2 = 0.461910218000412f;
-  constexpr float g3 = 0.05010765790939331f, g4 = -0.006412093993276358f;
-  constexpr float g5 = 0.00037955178413540125f;
-  const float ax = fabsf(x);
-  const float a = __builtin_amdgcn_fmed3f(ax, 0.0f, 5.0f);
-  float g = fmaf(g5, a, g4);
-  g = fmaf(g, a, g3);
-  g = fmaf(g, a, g2);
-  g = fmaf(g, a, g1);
-  g = fmaf(g, a, g0);
-  const float h = __builtin_amdgcn_exp2f(-g);
-  return fmaf(-ax, h, relu_bits(x));
-}
 
 SHRIMP_DEV u32x4 lds_frag(const unsigned char* wl, uint32_t base, int ks, int nb, int nbt,
                           int lane) {
@@ -343,21 +325,23 @@ __global__ void scale_rows_cols_kernel(const float* __restrict__ src, const floa
 using namespace shrimp;
 
 extern "C" size_t shrimp_attn_mlp_pack_bytes(int C, int hidden) {
+  if (block_stream_width(C) && hidden == 2 * C) return mlp_stream_pack_bytes(C);
   return (C == MC && hidden == MH) ? (size_t)PACK_BYTES : 0;
 }
 
 extern "C" int shrimp_pack_attn_mlp(const shrimp_mlp_weights* w, void* packed, void* scratch,
                                     void* stream) {
   SHRIMP_REQUIRE(w && packed && scratch, "pack_attn_mlp: null pointer");
-  SHRIMP_REQUIRE(w->C == MC && w->hidden == MH,
-                 "pack_attn_mlp: fused kernel covers C=%d, hidden=%d (got %d, %d)", MC, MH, w->C,
-                 w->hidden);
+  SHRIMP_REQUIRE(shrimp_attn_mlp_pack_bytes(w->C, w->hidden) > 0,
+                 "pack_attn_mlp: fused kernels cover C=%d, 96 and 192, hidden 2C (got %d, %d)", MC,
+                 w->C, w->hidden);
   SHRIMP_REQUIRE(w->out_w && w->out_b && w->g_attn && w->ln_w && w->ln_b && w->fc1_w &&
                      w->fc1_b && w->fc2_w && w->fc2_b && w->g_mlp,
                  "pack_attn_mlp: null weight pointer");
   hipStream_t st = as_stream(stream);
   unsigned char* pk = static_cast<unsigned char*>(packed);
-  float* tmp = static_cast<float*>(scratch);  // MC * MH floats
+  float* tmp = static_cast<float*>(scratch);  // C * hidden floats
+  if (w->C != MC) return pack_mlp_stream(w, pk, tmp, st);
   struct Part {
     const float* src; const float* rs; const float* cs; int n_out, n_in; uint32_t off; int il;
   } parts[3] = {{w->out_w, w->g_attn, nullptr, MC, MC, WO_OFF, 0},
@@ -381,22 +365,24 @@ extern "C" int shrimp_attn_mlp(const shrimp_mlp_args* a, void* stream) {
   SHRIMP_REQUIRE(a != nullptr, "attn_mlp: null args");
   SHRIMP_REQUIRE(a->rows >= 0, "attn_mlp: negative rows");
   if (a->rows == 0) return SHRIMP_OK;
-  SHRIMP_REQUIRE(a->C == MC && a->hidden == MH,
-                 "attn_mlp: fused kernel covers C=%d, hidden=%d (got C=%d, hidden=%d)", MC, MH,
-                 a->C, a->hidden);
+  const int C = a->C;
+  SHRIMP_REQUIRE(shrimp_attn_mlp_pack_bytes(C, a->hidden) > 0,
+                 "attn_mlp: fused kernels cover C=%d, 96 and 192, hidden 2C (got C=%d, hidden=%d)",
+                 MC, C, a->hidden);
   SHRIMP_REQUIRE(a->x && a->seq && a->mask && a->packed, "attn_mlp: null pointer");
   SHRIMP_REQUIRE(strides_ok({a->x_sr, a->s_sr}), "attn_mlp: row strides outside [0, 2^31)");
-  SHRIMP_REQUIRE(a->x_sr >= MC && a->x_sr % 8 == 0 && a->s_sr >= MC && a->s_sr % 8 == 0,
+  SHRIMP_REQUIRE(a->x_sr >= C && a->x_sr % 8 == 0 && a->s_sr >= C && a->s_sr % 8 == 0,
                  "attn_mlp: row strides must be >= C and multiples of 8");
-  const int64_t xe = ((int64_t)(a->rows - 1) * a->x_sr + MC) * 2;
-  const int64_t se = ((int64_t)(a->rows - 1) * a->s_sr + MC) * 2;
+  const int64_t xe = ((int64_t)(a->rows - 1) * a->x_sr + C) * 2;
+  const int64_t se = ((int64_t)(a->rows - 1) * a->s_sr + C) * 2;
   SHRIMP_REQUIRE(xe < (int64_t)0x7FFF0000 && se < (int64_t)0x7FFF0000,
                  "attn_mlp: activation buffer too large");
   SHRIMP_REQUIRE(a->S > 0 && a->rows % a->S == 0 && a->n_tokens >= 0 && a->n_tokens <= a->S,
                  "attn_mlp: rows must be whole positions of S rows (rows %d, S %d, tokens %d)",
                  a->rows, a->S, a->n_tokens);
-  const int64_t lob = a->tok_lo ? (int64_t)(a->rows / a->S) * a->n_tokens * MC * 2 : 0;
+  const int64_t lob = a->tok_lo ? (int64_t)(a->rows / a->S) * a->n_tokens * C * 2 : 0;
   SHRIMP_REQUIRE(lob < (int64_t)0x7FFF0000, "attn_mlp: token low parts too large");
+  if (C != MC) return launch_mlp_stream(a, (uint32_t)xe, (uint32_t)se, (uint32_t)lob, as_stream(stream));
   SHRIMP_REQUIRE((size_t)max_lds_per_block() >= W_LDS,
                  "attn_mlp: needs %u bytes of LDS per workgroup", (unsigned)W_LDS);
   int dev = 0, cus = 0;

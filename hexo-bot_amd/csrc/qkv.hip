@@ -26,6 +26,13 @@ __global__ void scale_rows_cols_kernel(const float* __restrict__ src, const floa
                                        const float* __restrict__ cs, int n_out, int n_in,
                                        float* __restrict__ dst);
 
+// 96 and 192 channels (block_stream.hip).
+bool block_stream_width(int C);
+size_t qkv_stream_pack_bytes(int C);
+int pack_qkv_stream(const float* w, const float* b, const float* ln_w, const float* ln_b,
+                    unsigned char* pk, float* tmp, int C, hipStream_t st);
+int launch_qkv_stream(const shrimp_qkv_args* a, uint32_t x_bytes, uint32_t q_bytes, hipStream_t st);
+
 namespace {
 
 constexpr int QC = QKV_C;                       // channels
@@ -209,15 +216,22 @@ __global__ void qkv_colsum_kernel(const unsigned short* __restrict__ frag, float
 
 using namespace shrimp;
 
-extern "C" size_t shrimp_attn_qkv_pack_bytes(int C) { return C == QC ? (size_t)QPACK_BYTES : 0; }
+extern "C" size_t shrimp_attn_qkv_pack_bytes(int C) {
+  if (block_stream_width(C)) return qkv_stream_pack_bytes(C);
+  return C == QC ? (size_t)QPACK_BYTES : 0;
+}
 
 extern "C" int shrimp_pack_attn_qkv(const float* qkv_w, const float* qkv_b, const float* ln_w,
                                     const float* ln_b, void* packed, void* scratch, int C,
                                     void* stream) {
   SHRIMP_REQUIRE(qkv_w && qkv_b && ln_w && ln_b && packed && scratch,
                  "pack_attn_qkv: null pointer");
-  SHRIMP_REQUIRE(C == QC, "pack_attn_qkv: fused kernel covers C=%d (got %d)", QC, C);
+  SHRIMP_REQUIRE(shrimp_attn_qkv_pack_bytes(C) > 0,
+                 "pack_attn_qkv: fused kernels cover C=%d, 96 and 192 (got %d)", QC, C);
   hipStream_t st = as_stream(stream);
+  if (C != QC)
+    return pack_qkv_stream(qkv_w, qkv_b, ln_w, ln_b, static_cast<unsigned char*>(packed),
+                           static_cast<float*>(scratch), C, st);
   float* tmp = static_cast<float*>(scratch);  // 3C * C floats
   unsigned char* pk = static_cast<unsigned char*>(packed);
   const int64_t n = (int64_t)QN * QC;
@@ -238,19 +252,24 @@ extern "C" int shrimp_attn_qkv(const shrimp_qkv_args* a, void* stream) {
   SHRIMP_REQUIRE(a != nullptr, "attn_qkv: null args");
   SHRIMP_REQUIRE(a->rows >= 0, "attn_qkv: negative rows");
   if (a->rows == 0) return SHRIMP_OK;
-  SHRIMP_REQUIRE(a->C == QC, "attn_qkv: fused kernel covers C=%d (got %d)", QC, a->C);
+  const int C = a->C;
+  SHRIMP_REQUIRE(shrimp_attn_qkv_pack_bytes(C) > 0,
+                 "attn_qkv: fused kernels cover C=%d, 96 and 192 (got %d)", QC, C);
   SHRIMP_REQUIRE(a->x && a->qkv && a->packed, "attn_qkv: null pointer");
   SHRIMP_REQUIRE(a->B > 0 && a->S > 0 && (int64_t)a->B * a->S == a->rows,
                  "attn_qkv: rows must be B * S");
-  SHRIMP_REQUIRE(a->H > 0 && QC % a->H == 0, "attn_qkv: C %% H != 0");
-  const int d = QC / a->H;
-  SHRIMP_REQUIRE(d >= 4 && (d & (d - 1)) == 0 && a->dpad >= d && a->dpad % 4 == 0,
-                 "attn_qkv: head dim %d must be a power of two >= 4 with dpad %d >= d", d, a->dpad);
-  SHRIMP_REQUIRE(strides_ok({a->x_sr}) && a->x_sr >= QC && a->x_sr % 8 == 0, "attn_qkv: x row stride");
-  const int64_t xe = ((int64_t)(a->rows - 1) * a->x_sr + QC) * 2;
+  SHRIMP_REQUIRE(a->H > 0 && C % a->H == 0, "attn_qkv: C %% H != 0");
+  const int d = C / a->H;
+  SHRIMP_REQUIRE(d >= 4 && (C == QC ? (d & (d - 1)) == 0 : d % 4 == 0) && a->dpad >= d &&
+                     a->dpad % 4 == 0,
+                 "attn_qkv: head dim %d must be a power of two >= 4 (96 and 192 channels: a "
+                 "multiple of 4) with dpad %d >= d", d, a->dpad);
+  SHRIMP_REQUIRE(strides_ok({a->x_sr}) && a->x_sr >= C && a->x_sr % 8 == 0, "attn_qkv: x row stride");
+  const int64_t xe = ((int64_t)(a->rows - 1) * a->x_sr + C) * 2;
   SHRIMP_REQUIRE(xe < (int64_t)0x7FFF0000, "attn_qkv: activation buffer too large");
   const int64_t qe = mul_sat({3, a->B, a->H, a->S, a->dpad, 2});  // q, k and v planes
   SHRIMP_REQUIRE(qe < (int64_t)0x7FFF0000, "attn_qkv: q/k/v buffer too large");
+  if (C != QC) return launch_qkv_stream(a, (uint32_t)xe, (uint32_t)qe, as_stream(stream));
   SHRIMP_REQUIRE((size_t)max_lds_per_block() >= QW_LDS, "attn_qkv: needs %u bytes of LDS",
                  (unsigned)QW_LDS);
   int dev = 0, cus = 0;

@@ -630,7 +630,8 @@ class HipForward:
         attn_fused = (P.fused_qkv and self.use_fused_qkv and self.use_fused_attn
                       and attn_fused_supported(C, H, S, dpad))
         staged = (not attn_fused and P.fused_qkv and self.use_fused_qkv and self.use_staged_attn
-                  and self.use_linear_bias and d == dpad and attn_staged_supported(H, S, dpad))
+                  and self.use_linear_bias and C == 128 and d == dpad
+                  and attn_staged_supported(H, S, dpad))
         qkv = kvf = meta = None
         if staged:
             sp = (S + 15) // 16 * 16
@@ -638,7 +639,10 @@ class HipForward:
             kvf = torch.empty((B, H, 2, sp, 16), dtype=bf, device=dev)
             meta = torch.empty((B, attn_keys_ints(S)), dtype=torch.int32, device=dev)
         elif not attn_fused:
-            qkv = (torch.zeros if d != dpad else torch.empty)((3, B, H, S, dpad), dtype=bf, device=dev)
+            # the padded channels are read: the fused q/k/v kernel of 96 and 192
+            # channels writes their zeros, the others leave them
+            fills = d == dpad or (P.fused_qkv and self.use_fused_qkv and C in (96, 192))
+            qkv = (torch.empty if fills else torch.zeros)((3, B, H, S, dpad), dtype=bf, device=dev)
         att = torch.empty((B, S, C), dtype=bf, device=dev)
         fused = P.fused_mlp and self.use_fused_mlp
         hid = None if fused else torch.empty((B, S, 2 * C), dtype=bf, device=dev)

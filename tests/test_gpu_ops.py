@@ -1362,3 +1362,61 @@ def test_conv_weight_streamed(cin, c, B, N):
     close(got[3], want, what="LN + ReLU")
     for k, (a, b) in enumerate(zip(got, run(1))):
         assert torch.equal(a, b), k
+
+
+# the weight-streamed row kernels of the attention block at 96 and 192 channels: a
+# single position shorter than one wave's rows, a ragged last tile and both row
+# tilings (16 rows per wave below 128 rows per compute unit, 32 from there);
+# head dims with and without padded channels (which the kernel zeroes)
+@pytest.mark.parametrize("B,S", [(1, 9), (3, 43), (131, 257)])
+@pytest.mark.parametrize("c,H", [(96, 4), (192, 3), (192, 8)])
+def test_block_rows_weight_streamed(c, H, B, S):
+    from shrimp import ops
+
+    g = torch.Generator().manual_seed(B * S + c + H)
+    rows, hid, nt = B * S, 2 * c, 8
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g) * std
+    x, seq, lo = r(rows, c), r(rows, c), r(B, nt, c, std=2.0 ** -10)
+    m = torch.rand(rows, generator=g) < 0.8
+    wq, bq = r(3 * c, c, std=0.08), r(3 * c, std=0.1)
+    lnw, lnb = torch.rand(c, generator=g) + 0.5, r(c, std=0.1)
+    wo, bo, w1, b1 = r(c, c, std=0.08), r(c, std=0.1), r(hid, c, std=0.08), r(hid, std=0.1)
+    w2, b2 = r(c, hid, std=0.06), r(c, std=0.1)
+    ga, gm = torch.rand(c, generator=g) * 0.5 + 0.5, torch.rand(c, generator=g) * 0.5 + 0.5
+    dv = lambda t: t.to(DEV)
+    d, D = c // H, lambda t: t.double()
+    dpad = max(16, -(-d // 16) * 16)
+    F = torch.nn.functional
+
+    seq_d = dv(seq).to(torch.bfloat16)
+    qkv = torch.full((3, B, H, S, dpad), 7.0, dtype=torch.bfloat16, device=DEV)
+    packed = ops.pack_attn_qkv(dv(wq), dv(bq), dv(lnw), dv(lnb))
+    ops.launch_attn_qkv(x=seq_d, x_sr=c, qkv=qkv, packed=packed, eps=1e-5, rows=rows, B=B, S=S, H=H,
+                        C=c, dpad=dpad)
+    n = F.layer_norm(bf(seq), (c,), D(lnw), D(lnb), 1e-5)
+    want = (n @ D(wq).T + D(bq)).reshape(B, S, 3, H, d).permute(2, 0, 3, 1, 4)
+    # bf16 operands: sqrt(c) products of relative error 2^-8 around |n| |w|, and bf16 out
+    close(qkv[..., :d], want, atol=4e-2, rtol=1e-2, what="qkv")
+    assert (qkv[..., d:] == 0).all()
+
+    lo_d = dv(lo).to(torch.bfloat16)
+    packed = ops.pack_attn_mlp(*(dv(t) for t in (wo, bo, ga, lnw, lnb, w1, b1, w2, b2, gm)))
+    ops.launch_attn_mlp(x=dv(x).to(torch.bfloat16), x_sr=c, seq=seq_d, s_sr=c,
+                        mask=dv(m).to(torch.uint8), packed=packed, eps=1e-5, rows=rows, C=c,
+                        hidden=hid, tok_lo=lo_d, S=S, n_tokens=nt)
+    full = bf(seq).reshape(B, S, c).clone()
+    full[:, :nt] += bf(lo)
+    full = full.reshape(rows, c)
+    mm = D(m)[:, None]
+    s1 = full + D(ga) * ((bf(x) @ D(wo).T + D(bo)) * mm)
+    h = F.gelu(F.layer_norm(s1, (c,), D(lnw), D(lnb), 1e-5) @ D(w1).T + D(b1))
+    want = s1 + D(gm) * ((h @ D(w2).T + D(b2)) * mm)
+    close(seq_d, want, atol=5e-2, rtol=1e-2, what="mlp")
+    # masked rows keep their residual; live token rows keep 16 significant bits
+    got = seq_d.cpu().double().reshape(B, S, c)
+    keep = (~m).reshape(B, S)
+    assert torch.equal(got[keep], bf(seq).reshape(B, S, c)[keep])
+    tok = got[:, :nt] + lo_d.cpu().double()
+    low = (tok - got[:, :nt]).abs() <= 2.0 ** -8 * got[:, :nt].abs() + 1e-6
+    assert low[~keep[:, :nt]].all()
+    assert torch.equal(lo_d.cpu().double()[keep[:, :nt]], bf(lo)[keep[:, :nt]])

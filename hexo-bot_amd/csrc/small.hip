@@ -92,6 +92,109 @@ constexpr int PREP_FEAT = 4, PREP_IDX = 2, PREP_PARTS = PREP_FEAT + PREP_IDX + 1
 // prep_csr_kernel spreads its flat loops over PREP_CSR_PARTS workgroups per row
 constexpr int PREP_CSR_PARTS = 4;
 
+// ---- operand preparation of the operator entry points ---------------------------
+// Everything an operator call converts (row dtype and channel padding, int64
+// indices, the weight's fragment order) in one launch: a table of up to
+// OP_JOBS jobs, each over its own range of workgroups. Three to five library
+// launches of a few microseconds each stood before the kernel.
+constexpr int OP_JOBS = 6;
+enum : int { OP_ROWS_BF16 = 0, OP_INDEX_I32 = 1, OP_CONV_W_BF16 = 2, OP_RAYTAP_W_F16 = 3 };
+
+struct OpJob {
+  const void* src;
+  void* dst;
+  int op, dt;
+  int64_t n;      // work items: 8 row elements, 4 indices, or one lane's 8 weights
+  int width, dst_width, extra;
+  int blocks;     // workgroups of 256 items
+  bool vec;       // 16-byte source loads
+};
+struct OpJobs {
+  OpJob j[OP_JOBS];
+};
+
+template <int DT>
+SHRIMP_DEV void op_rows(const OpJob& j, int64_t i) {
+  float v[8];
+  const int64_t e0 = i * 8;
+  if (j.vec) {  // whole rows copied element for element
+    if constexpr (DT == SHRIMP_DT_F32) {
+      const f32x4* s = reinterpret_cast<const f32x4*>(static_cast<const float*>(j.src) + e0);
+      const f32x4 a = s[0], b = s[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+      }
+    } else {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(j.src) + e0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned short h = (unsigned short)(a[e >> 1] >> (16 * (e & 1)));
+        if constexpr (DT == SHRIMP_DT_F16) v[e] = (float)__builtin_bit_cast(_Float16, h);
+        else v[e] = bf16_bits_to_f32(h);
+      }
+    }
+  } else {
+    const int64_t row = e0 / j.dst_width;  // dst_width % 8 == 0: one row
+    const int c0 = (int)(e0 - row * j.dst_width);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = c0 + e < j.width ? load_feat_t<DT>(j.src, row * j.width + c0 + e) : 0.f;
+  }
+  *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(j.dst) + e0) =
+      u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+            pack_bf16x2(v[6], v[7])};
+}
+
+__global__ __launch_bounds__(256) void op_prep_kernel(const OpJobs jobs, int n_jobs) {
+  int blk = (int)blockIdx.x, k = 0;
+  while (k + 1 < n_jobs && blk >= jobs.j[k].blocks) blk -= jobs.j[k++].blocks;  // uniform
+  const OpJob& j = jobs.j[k];
+  const int64_t i = (int64_t)blk * 256 + threadIdx.x;
+  if (i >= j.n) return;
+  if (j.op == OP_ROWS_BF16) {
+    if (j.dt == SHRIMP_DT_F32) op_rows<SHRIMP_DT_F32>(j, i);
+    else if (j.dt == SHRIMP_DT_F16) op_rows<SHRIMP_DT_F16>(j, i);
+    else op_rows<SHRIMP_DT_BF16>(j, i);
+  } else if (j.op == OP_INDEX_I32) {
+    // four indices per item; `width` of them exist in the last
+    const int64_t* s = static_cast<const int64_t*>(j.src) + i * 4;
+    int32_t* d = static_cast<int32_t*>(j.dst) + i * 4;
+    if (i + 1 < j.n || j.width == 4) {
+      const int64_t v[4] = {s[0], s[1], s[2], s[3]};
+      *reinterpret_cast<int4*>(d) = int4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+    } else {
+      for (int e = 0; e < j.width; ++e) d[e] = (int32_t)s[e];
+    }
+  } else {
+    // fragment i / 64 = (K step) NB + output block, lane i % 64: eight inputs of
+    // one output; K = tap dst_width + channel, weights (tap, channel, output) fp32
+    const int lane = (int)(i & 63), NB = j.extra / 16;
+    const int64_t f = i >> 6;
+    const int nb = (int)(f % NB), ks = (int)(f / NB);
+    const int n = nb * 16 + (lane & 15), k0 = ks * 32 + (lane >> 4) * 8;
+    const float* w = static_cast<const float*>(j.src);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int t = (k0 + e) / j.dst_width, c = (k0 + e) - t * j.dst_width;
+      v[e] = c < j.width ? w[((int64_t)t * j.width + c) * j.extra + n] : 0.f;
+    }
+    u32x4 o;
+    if (j.op == OP_CONV_W_BF16) {
+      o = u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                pack_bf16x2(v[6], v[7])};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = (unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * e]) |
+               ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * e + 1]) << 16);
+    }
+    *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(j.dst) + i * 8) = o;
+  }
+}
+
 // ---- input preparation (model.py:861-863, 884-892; batching.py:264-276) --------
 // Each output array is written by a flat loop over its elements, so
 // consecutive lanes touch consecutive addresses. The pointers are __restrict__
@@ -629,6 +732,57 @@ __global__ __launch_bounds__(256) void ray_index_kernel(const int32_t* coords, c
 }  // namespace shrimp
 
 using namespace shrimp;
+
+extern "C" int shrimp_op_prep(const int64_t* words, int n_jobs, void* stream) {
+  SHRIMP_REQUIRE(n_jobs >= 0 && n_jobs <= OP_JOBS, "op_prep: %d jobs, at most %d", n_jobs, OP_JOBS);
+  SHRIMP_REQUIRE(n_jobs == 0 || words, "op_prep: null jobs");
+  OpJobs jobs{};
+  int64_t blocks = 0;
+  int k = 0;
+  for (int i = 0; i < n_jobs; ++i, words += 8) {
+    OpJob j{};
+    j.src = reinterpret_cast<const void*>((uintptr_t)words[0]);
+    j.dst = reinterpret_cast<void*>((uintptr_t)words[1]);
+    const int64_t op = words[2], dt = words[3], rows = words[4], width = words[5], dw = words[6],
+                  extra = words[7];
+    SHRIMP_REQUIRE(rows >= 0 && rows < ((int64_t)1 << 40), "op_prep: bad row count");
+    if (rows == 0) continue;
+    SHRIMP_REQUIRE(j.src && j.dst && (words[1] & 15) == 0, "op_prep: null or unaligned pointer");
+    j.op = (int)op;
+    j.dt = (int)dt;
+    if (op == OP_ROWS_BF16) {
+      SHRIMP_REQUIRE(dt == SHRIMP_DT_F32 || dt == SHRIMP_DT_F16 || dt == SHRIMP_DT_BF16,
+                     "op_prep: rows of dtype %d", (int)dt);
+      SHRIMP_REQUIRE(width > 0 && width <= dw && dw <= kMaxDim && dw % 8 == 0,
+                     "op_prep: %lld channels padded to %lld (a multiple of 8)", (long long)width,
+                     (long long)dw);
+      j.vec = width == dw && (words[0] & 15) == 0;
+      j.n = rows * (dw / 8);
+    } else if (op == OP_INDEX_I32) {
+      SHRIMP_REQUIRE(dt == SHRIMP_DT_I64 && (words[0] & 7) == 0, "op_prep: indices of dtype %d", (int)dt);
+      j.n = (rows + 3) / 4;
+    } else {
+      SHRIMP_REQUIRE((op == OP_CONV_W_BF16 || op == OP_RAYTAP_W_F16) && dt == SHRIMP_DT_F32,
+                     "op_prep: unknown job %lld of dtype %d", (long long)op, (int)dt);
+      SHRIMP_REQUIRE(rows <= 64 && width > 0 && width <= dw && dw % 32 == 0 && extra > 0 &&
+                         extra % 16 == 0 && mul_sat({rows, dw, extra, 2}) < (int64_t)0x7FFF0000,
+                     "op_prep: weight (%lld, %lld -> %lld, %lld)", (long long)rows, (long long)width,
+                     (long long)dw, (long long)extra);
+      j.n = rows * dw * extra / 8;
+    }
+    j.width = op == OP_INDEX_I32 ? (int)(rows - (j.n - 1) * 4) : (int)width;
+    j.dst_width = (int)dw;
+    j.extra = (int)extra;
+    const int64_t nb = (j.n + 255) / 256;
+    blocks += nb;
+    SHRIMP_REQUIRE(blocks < ((int64_t)1 << 31), "op_prep: too large");
+    j.blocks = (int)nb;
+    jobs.j[k++] = j;
+  }
+  if (k == 0) return SHRIMP_OK;
+  hipLaunchKernelGGL(op_prep_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), jobs, k);
+  return check_launch("op_prep");
+}
 
 extern "C" int shrimp_prep_inputs(const void* nbr, int nbr_dt, const void* mask, const void* coords,
                                   int coords_dt, const void* feats, int feats_dt, int nfeat, int B,

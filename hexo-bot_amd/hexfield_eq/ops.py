@@ -16,7 +16,7 @@ import functools
 import torch
 
 from shrimp import _lib
-from shrimp.ops import require_device
+from shrimp.ops import mask_bytes, require_device
 
 RAY_GATHER_SLOTS = 32
 RAY_REACH = 5
@@ -152,6 +152,20 @@ def pack_raytap_weight(weight: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _packed_weight(weight: torch.Tensor) -> torch.Tensor:
+    """pack_raytap_weight, an fp32 weight rounded and packed in one launch."""
+
+    t, c, cout = weight.shape
+    nbytes = _load().shrimp_raytap_wpack_bytes(c, cout)
+    if weight.dtype != torch.float32 or t != 7 or nbytes == 0:
+        return pack_raytap_weight(weight)
+    w = weight.detach().contiguous()
+    out = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
+    _lib.op_prep([(w.data_ptr(), out.data_ptr(), _lib.PREP_RAYTAP_W, _lib.DT_F32, t, c, c, cout)],
+                 _lib.stream_handle(w.device))
+    return out
+
+
 def launch_conv_ln_raytap(x, gidx32, mask8, packed, bias32, lnw32, lnb32, ray_idx32, reach8,
                           alpha16, eps, relu, corb, out) -> None:
     """Raw launch of K1 on prepared buffers (see the header for layouts)."""
@@ -263,17 +277,22 @@ def hex_conv_ln_raytap(
     b, n, c = x.shape
     cout = weight.shape[-1]
     xh = _fp16_view(x)
-    gi = gather_idx.to(torch.int32)
-    if gi.stride(-1) != 1:
-        gi = gi.contiguous()
-    m8 = mask.to(torch.uint8).contiguous()
+    gi = gather_idx
+    if gi.dtype == torch.int64:
+        # only slot 0 is read: the low dwords of the int64 indices in place
+        gi = (gi if gi.stride(-1) == 1 else gi.contiguous()).view(torch.int32)
+    else:
+        gi = gi.to(torch.int32)
+        if gi.stride(-1) != 1:
+            gi = gi.contiguous()
+    m8 = mask_bytes(mask)
     ri = ray_idx.to(torch.int32)
     if ri.stride(-1) != 1:
         ri = ri.contiguous()
     re = reach.to(torch.uint8).reshape(b, n, 12)
     if re.stride(-1) != 1:
         re = re.contiguous()
-    packed = pack_raytap_weight(weight.reshape(7, c, cout))
+    packed = _packed_weight(weight.reshape(7, c, cout))
     out = torch.empty((b, n, cout), dtype=torch.float16, device=x.device)
     launch_conv_ln_raytap(
         xh, gi, m8, packed, bias.to(torch.float32).contiguous(),

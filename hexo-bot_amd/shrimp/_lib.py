@@ -145,6 +145,7 @@ SIGNATURES: dict = {
     "shrimp_max_lds_per_block": (ctypes.c_int, []),
     "shrimp_conv_wpack_bytes": (ctypes.c_size_t, [ctypes.c_int] * 3),
     "shrimp_pack_conv_weight": (ctypes.c_int, [_vp, _vp] + [ctypes.c_int] * 4 + [_vp]),
+    "shrimp_op_prep": (ctypes.c_int, [ctypes.POINTER(_i64), ctypes.c_int, _vp]),
     "shrimp_linear_wpack_bytes": (ctypes.c_size_t, [ctypes.c_int] * 2),
     "shrimp_pack_linear_weight": (ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.c_int, _vp]),
     "shrimp_hex_conv": (ctypes.c_int, [ctypes.POINTER(ConvArgs), _vp]),
@@ -259,6 +260,18 @@ def check(status: int, what: str) -> None:
     if status != 0:
         msg = load().shrimp_last_error()
         raise RuntimeError(f"{what} failed ({status}): {msg.decode() if msg else ''}")
+
+
+PREP_ROWS_BF16, PREP_INDEX_I32, PREP_CONV_W, PREP_RAYTAP_W = range(4)
+
+
+def op_prep(jobs: list, stream: int) -> None:
+    """shrimp_op_prep: (src, dst, op, src dtype, rows, width, dst_width, extra)
+    per job, in one launch."""
+
+    if jobs:
+        words = (_i64 * (8 * len(jobs)))(*(w for j in jobs for w in j))
+        check(load().shrimp_op_prep(words, len(jobs), stream), "op_prep")
 
 
 def ptr(t) -> int | None:

@@ -419,35 +419,71 @@ def ctypes_ref(struct):
 # ---- the reference operator ABI -----------------------------------------------------------
 
 
-def _bf16_rows(x: torch.Tensor, cin_pad: int) -> torch.Tensor:
-    """x (B, N, C) -> contiguous bf16 (B, N, cin_pad) (zero channel padding)."""
+_ROW_DT = {
+    torch.float32: _lib.DT_F32,
+    torch.float16: _lib.DT_F16,
+    torch.bfloat16: _lib.DT_BF16,
+}
 
-    b, n, c = x.shape
-    xb = x.to(torch.bfloat16)
-    if c == cin_pad:
-        return xb.contiguous()
-    out = torch.zeros((b, n, cin_pad), dtype=torch.bfloat16, device=x.device)
-    out[..., :c] = xb
+
+def prep_rows(t: torch.Tensor, pad: int, jobs: list) -> torch.Tensor:
+    """t (..., C) as contiguous bf16 rows of ``pad`` channels (zeros past C): t
+    itself, or a tensor that a job of ``jobs`` (_lib.op_prep) fills."""
+
+    c = t.shape[-1]
+    if t.dtype == torch.bfloat16 and c == pad and t.is_contiguous():
+        return t
+    if t.dtype not in _ROW_DT:
+        t = t.to(torch.bfloat16)
+    t = t.contiguous()
+    out = torch.empty((*t.shape[:-1], pad), dtype=torch.bfloat16, device=t.device)
+    jobs.append((t.data_ptr(), out.data_ptr(), _lib.PREP_ROWS_BF16, _ROW_DT[t.dtype],
+                 t.numel() // c if c else 0, c, pad, 0))
+    out._prep_source = t  # converted on the stream later: not freed before the launch
     return out
+
+
+def prep_index(t: torch.Tensor, jobs: list) -> torch.Tensor:
+    """t as contiguous int32: t itself, or a tensor that a job fills (int64)."""
+
+    if t.dtype != torch.int64:
+        return t.to(torch.int32).contiguous()
+    t = t.contiguous()
+    out = torch.empty(t.shape, dtype=torch.int32, device=t.device)
+    jobs.append((t.data_ptr(), out.data_ptr(), _lib.PREP_INDEX_I32, _lib.DT_I64, t.numel(), 0, 0, 0))
+    out._prep_source = t
+    return out
+
+
+def mask_bytes(mask: torch.Tensor) -> torch.Tensor:
+    """mask as contiguous uint8 (a bool tensor's bytes are 0 and 1 already)."""
+
+    mask = mask.contiguous()
+    return mask.view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8)
 
 
 def _conv_common(x, gather_idx, mask, weight, bias, ln_weight, ln_bias, eps, relu):
     require_device(x, "shrimp::hex_conv")
     b, n, c = x.shape
-    t = weight.shape[0]
-    cout = weight.shape[-1]
+    t, cin, cout = weight.shape
     cp = cin_pad_of(c)
-    xb = _bf16_rows(x, cp)
-    idx = gather_idx.to(torch.int32).contiguous()
-    m8 = mask.to(torch.uint8).contiguous()
-    wp = pack_conv_weight(weight, cp)
+    jobs = []
+    xb = prep_rows(x, cp, jobs)
+    idx = prep_index(gather_idx, jobs)
+    m8 = mask_bytes(mask)
+    w32 = weight.detach().to(torch.float32).contiguous()
+    wp = torch.empty(_lib.load().shrimp_conv_wpack_bytes(t, cp, cout), dtype=torch.uint8,
+                     device=weight.device)
+    jobs.append((w32.data_ptr(), wp.data_ptr(), _lib.PREP_CONV_W, _lib.DT_F32, t, cin, cp, cout))
+    st = _lib.stream_handle(x.device)
+    _lib.op_prep(jobs, st)
     out = torch.empty((b, n, cout), dtype=torch.bfloat16, device=x.device)
     launch_conv(
         x=xb, x_sb=n * cp, x_sn=cp, idx=idx, taps=t, idx_stride=idx.shape[-1], mask8=m8,
         wpack=wp, bias=bias.to(torch.float32).contiguous(), B=b, N=n, cin_pad=cp, cout=cout,
         ln_w=None if ln_weight is None else ln_weight.to(torch.float32).contiguous(),
         ln_b=None if ln_bias is None else ln_bias.to(torch.float32).contiguous(),
-        eps=eps, relu=relu, out=out, o_sb=n * cout, o_sn=cout,
+        eps=eps, relu=relu, out=out, o_sb=n * cout, o_sn=cout, stream=st,
     )
     return out
 
@@ -511,13 +547,10 @@ def attn_pair(
     b, h, s, d = q.shape
     dpad = max(16, -(-d // 16) * 16)
 
-    def prep(t):
-        t = t.to(torch.bfloat16)
-        if dpad != d:
-            t = torch.nn.functional.pad(t, (0, dpad - d))
-        return t.contiguous()
-
-    qb, kb, vb = prep(q), prep(k), prep(v)
+    jobs = []
+    qb, kb, vb = (prep_rows(t, dpad, jobs) for t in (q, k, v))
+    st = _lib.stream_handle(q.device)
+    _lib.op_prep(jobs, st)
     pr = pair.to(torch.uint8).contiguous()
     tab = table2.to(torch.float32).contiguous()
     sl = seq_lens.to(torch.int32).contiguous()
@@ -525,7 +558,7 @@ def attn_pair(
     launch_attn(
         q=qb, k=kb, v=vb, qkv_sb=h * s * dpad, qkv_sh=s * dpad, seq_lens=sl,
         o=out, o_sb=h * s * d, o_sh=s * d, o_sr=d, B=b, S=s, H=h, d=d, dpad=dpad,
-        pair=pr, p_sb=s * s, p_sq=s, table2=tab, n_tokens=0,
+        pair=pr, p_sb=s * s, p_sq=s, table2=tab, n_tokens=0, stream=st,
     )
     return out
 

@@ -101,6 +101,18 @@ size_t shrimp_linear_wpack_bytes(int in_features, int out_features);
 int shrimp_pack_linear_weight(const float* w, void* packed, int in_features, int out_features,
                               void* stream);
 
+/* Operand conversions of one operator call in one launch: n_jobs <= 6 jobs of
+ * eight int64 words each (host memory, read before the call returns):
+ *   {src, dst, op, src dtype, rows, width, dst_width, extra}
+ *   op 0  rows (rows, width) fp32 / fp16 / bf16, contiguous -> (rows,
+ *         dst_width) bf16, zeros past width; dst_width % 8 == 0
+ *   op 1  `rows` int64 indices -> int32 (low 32 bits)
+ *   op 2  conv weight (rows taps, width, extra) fp32 -> the packed layout of
+ *         shrimp_pack_conv_weight with cin_pad = dst_width
+ *   op 3  the same weight rounded to fp16, as shrimp_pack_raytap_weight packs it
+ * dst is 16-byte aligned. */
+int shrimp_op_prep(const int64_t* jobs, int n_jobs, void* stream);
+
 /* ------------------------------------------------------------------------
  * Gather-GEMM hex / ray-tap convolution with fused epilogue.
  *

@@ -1420,3 +1420,47 @@ def test_block_rows_weight_streamed(c, H, B, S):
     low = (tok - got[:, :nt]).abs() <= 2.0 ** -8 * got[:, :nt].abs() + 1e-6
     assert low[~keep[:, :nt]].all()
     assert torch.equal(lo_d.cpu().double()[keep[:, :nt]], bf(lo)[keep[:, :nt]])
+
+
+# every operand conversion of the operator calls in one launch: vector and
+# element loads (padded channels, a source off 16 bytes), tails of the index and
+# of a workgroup, both weight layouts, six jobs at once, no rows; special values
+# round as torch rounds them
+def test_op_prep_matches_torch():
+    from hexfield_eq import ops as hops
+    from shrimp import _lib, ops
+
+    g = torch.Generator().manual_seed(3)
+    st = _lib.stream_handle()
+    special = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), 1e38, 6e4, 1e-40, 65504.0])
+    for n, c, pad in ((1, 8, 8), (37, 96, 96), (5, 15, 32), (300, 24, 32), (3, 64, 64)):
+        x = torch.randn(n, c, generator=g)
+        x.view(-1)[:8] = special
+        jobs, outs, wants = [], [], []
+        for dt in (torch.float32, torch.float16, torch.bfloat16):
+            t = x.to(DEV, dt)
+            off = torch.empty(t.numel() + 1, dtype=dt, device=DEV)[1:].view(n, c).copy_(t)
+            for s in (t, off):
+                outs.append(ops.prep_rows(s, pad, jobs))
+                wants.append(torch.nn.functional.pad(s.to(torch.bfloat16), (0, pad - c)))
+        _lib.op_prep(jobs, st)
+        for o, w in zip(outs, wants):
+            assert torch.equal(o.cpu(), w.cpu())
+    for n in (1, 3, 4, 1021, 4096):
+        jobs, i = [], torch.randint(-(1 << 40), 1 << 40, (n,), generator=g).to(DEV)
+        o = ops.prep_index(i, jobs)
+        _lib.op_prep(jobs, st)
+        assert torch.equal(o, i.to(torch.int32))
+    for t, cin, cp, cout in ((7, 15, 32, 96), (31, 128, 128, 128), (7, 96, 96, 192)):
+        w = torch.randn(t, cin, cout, generator=g).to(DEV)
+        want = ops.pack_conv_weight(w, cp)
+        o = torch.empty_like(want)
+        _lib.op_prep([(w.data_ptr(), o.data_ptr(), _lib.PREP_CONV_W, _lib.DT_F32, t, cin, cp, cout)], st)
+        assert torch.equal(o, want)
+    w = torch.randn(7, 64, 96, generator=g).to(DEV)
+    assert torch.equal(hops._packed_weight(w), hops.pack_raytap_weight(w))
+    _lib.op_prep([], st)
+    for bad in ((0, 0, 0, 1, 4, 8, 8, 0), (w.data_ptr(), w.data_ptr(), 9, 1, 4, 8, 8, 0),
+                (w.data_ptr(), w.data_ptr(), 0, 1, 4, 8, 12, 0)):
+        with pytest.raises(RuntimeError, match="op_prep"):
+            _lib.op_prep([bad], st)

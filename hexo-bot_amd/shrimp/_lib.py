@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from pathlib import Path
 
 LIB_DIR = Path(__file__).resolve().parent / "_lib"
@@ -145,6 +146,8 @@ SIGNATURES: dict = {
     "shrimp_max_lds_per_block": (ctypes.c_int, []),
     "shrimp_conv_wpack_bytes": (ctypes.c_size_t, [ctypes.c_int] * 3),
     "shrimp_pack_conv_weight": (ctypes.c_int, [_vp, _vp] + [ctypes.c_int] * 4 + [_vp]),
+    "shrimp_forward_bytes": (_i64, [ctypes.POINTER(_i64)] + [ctypes.c_int] * 4),
+    "shrimp_forward": (ctypes.c_int, [ctypes.POINTER(_i64), ctypes.POINTER(_i64), _vp]),
     "shrimp_op_prep": (ctypes.c_int, [ctypes.POINTER(_i64), ctypes.c_int, _vp]),
     "shrimp_linear_wpack_bytes": (ctypes.c_size_t, [ctypes.c_int] * 2),
     "shrimp_pack_linear_weight": (ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.c_int, _vp]),
@@ -262,6 +265,19 @@ def check(status: int, what: str) -> None:
         raise RuntimeError(f"{what} failed ({status}): {msg.decode() if msg else ''}")
 
 
+FWD_STAGED, FWD_QKV, FWD_MLP, FWD_BLOCK, FWD_PAIR, FWD_TAIL, FWD_LINEAR_BIAS = (1 << i for i in range(7))
+
+
+def words(*values):
+    """int64 words for an entry point that takes them."""
+
+    return (_i64 * len(values))(*values)
+
+
+def float_word(x: float) -> int:
+    return int.from_bytes(struct.pack("<f", float(x)), "little")
+
+
 PREP_ROWS_BF16, PREP_INDEX_I32, PREP_CONV_W, PREP_RAYTAP_W = range(4)
 
 
@@ -270,8 +286,8 @@ def op_prep(jobs: list, stream: int) -> None:
     per job, in one launch."""
 
     if jobs:
-        words = (_i64 * (8 * len(jobs)))(*(w for j in jobs for w in j))
-        check(load().shrimp_op_prep(words, len(jobs), stream), "op_prep")
+        flat = words(*(w for j in jobs for w in j))
+        check(load().shrimp_op_prep(flat, len(jobs), stream), "op_prep")
 
 
 def ptr(t) -> int | None:

@@ -269,12 +269,14 @@ class ShrimpEvaluator:
         rt = self.model.hip_runtime()
         perf = self._perf.begin(compute) if self._perf is not None else None
         groups = plan_groups(sizes)
+        # looked up once per payload, packed on the compute stream before any side
+        # stream forks
+        packed = rt.weights(dev) if groups and not self.graphs else None
         side = []
         if not self.graphs and self.group_streams > 1 and len(groups) > 1:
             while len(self._group_streams) < self.group_streams:
                 self._group_streams.append(torch.cuda.Stream(dev))
             side = self._group_streams[: self.group_streams]
-            rt.weights(dev)  # packed on the compute stream, before the side streams fork
             slots = assign_group_streams(
                 [(e - s) * (p + NUM_TOKENS) ** 2 for s, e, p in groups], len(side))
             for s in side:
@@ -293,7 +295,8 @@ class ShrimpEvaluator:
                 out = rt.graph_forward_csr(*csr, start, g, pad_to, request_moves_left=request_ml) \
                     if self.graphs else None
                 if out is None:
-                    out = rt.forward_csr(*csr, start, g, pad_to, request_moves_left=request_ml)
+                    out = rt.forward_csr(*csr, start, g, pad_to, request_moves_left=request_ml,
+                                         packed=packed)
                 pol = out["policy"]
                 _lib.check(
                     lib.shrimp_decode(

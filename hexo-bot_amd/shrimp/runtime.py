@@ -203,9 +203,18 @@ class HipForward:
         # names it one way and tensors that name it the other would re-pack the
         # weights at every switch
         index = torch.cuda.current_device() if device.index is None else device.index
-        return (device.type, index, self.precision) + tuple(
-            (p.data_ptr(), p._version) for p in self.net.parameters()
-        )
+        # the module tree walked directly: net.parameters() builds a name and a
+        # set entry per parameter, 0.2 ms for a 12-block network
+        key = [device.type, index, self.precision]
+        todo = [self.net]
+        while todo:
+            m = todo.pop()
+            for p in m._parameters.values():
+                if p is not None:
+                    key.append(p.data_ptr())
+                    key.append(p._version)
+            todo.extend(m._modules.values())
+        return tuple(key)
 
     @property
     def fp32(self) -> bool:
@@ -284,6 +293,7 @@ class HipForward:
                                               CELL_LUT_M),
                 )
             )
+        P.words = None  # the network words of shrimp_forward (_net_words)
         P.fused_mlp = all(a.mlp is not None for a in P.attn)
         P.fused_qkv = all(a.qkv is not None for a in P.attn)
         P.tokens = f32(net.tokens)
@@ -303,6 +313,33 @@ class HipForward:
             hw=f32(net.policy_head.weight.reshape(-1)), hb=f32(net.policy_head.bias.reshape(-1)),
         )
         return P
+
+    @staticmethod
+    def _net_words(P):
+        """The packed network as shrimp_forward takes it (csrc/forward.cpp)."""
+
+        if P.words is None:
+            p, f = _lib.ptr, _lib.float_word
+            head = lambda h: [p(h.rw), p(h.rb), p(h.hw), p(h.hb)]
+            w = [len(P.layout), P.C, P.H, P.d, P.dpad, p(P.tokens), p(P.stem.w), p(P.stem.b),
+                 p(P.stem.lnw), p(P.stem.lnb), f(P.stem.eps), p(P.lnf.w), p(P.lnf.b), f(P.lnf.eps),
+                 *head(P.value), *head(P.ml), p(P.policy.w), p(P.policy.b), p(P.policy.hw),
+                 p(P.policy.hb), CELL_LUT_M, NUM_TOKENS, VALUE_BINS]
+            convs, attns = iter(P.convs), iter(P.attn)
+            for kind in P.layout:
+                if kind == "C":
+                    k = next(convs)
+                    layer = [0, p(k.w1), p(k.b1), p(k.ln1w), p(k.ln1b), f(k.eps1), p(k.w2), p(k.b2),
+                             p(k.ln2w), p(k.ln2b), f(k.eps2), p(k.gamma)]
+                else:
+                    a = next(attns)
+                    layer = [1, p(a.qkv), p(a.qkv_w), p(a.qkv_b), p(a.ln1w), p(a.ln1b), f(a.eps1),
+                             p(a.mlp), p(a.out_w), p(a.out_b), p(a.g_attn), p(a.ln2w), p(a.ln2b),
+                             f(a.eps2), p(a.fc1_w), p(a.fc1_b), p(a.fc2_w), p(a.fc2_b), p(a.g_mlp),
+                             p(a.btab_xtab[0]), p(a.btab_xtab[1])]
+                w += [x or 0 for x in layer] + [0] * (21 - len(layer))
+            P.words = _lib.words(*w)
+        return P.words
 
     @torch.no_grad()
     def _pack32(self, device: torch.device) -> SimpleNamespace:
@@ -408,11 +445,12 @@ class HipForward:
 
     @torch.no_grad()
     def forward_csr(self, node_feats, node_qr, nbr, row_offsets, row0: int, B: int, N: int, *,
-                    request_moves_left: bool = False) -> dict:
+                    request_moves_left: bool = False, packed=None) -> dict:
         """Forward over rows row0 .. row0 + B - 1 of ABI-1 payload arrays already on
         the device (node_feats (T, 15) f16, node_qr (T, 2) i16, nbr (T, 6) u16,
         row_offsets (rows + 1) int64), padded to N cells on the device
-        (inference.py:865-892 / serve_pack.rs:155-216 in one kernel)."""
+        (inference.py:865-892 / serve_pack.rs:155-216 in one kernel). ``packed``:
+        the result of ``weights`` for these rows' device, when the caller has it."""
 
         require_device(node_feats, "HipForward.forward_csr")
         dev = node_feats.device
@@ -428,14 +466,15 @@ class HipForward:
         lim = self.batch_limit(N)
         if B > lim:
             parts = [self.forward_csr(node_feats, node_qr, nbr, row_offsets, row0 + i,
-                                      min(lim, B - i), N, request_moves_left=request_moves_left)
+                                      min(lim, B - i), N, request_moves_left=request_moves_left,
+                                      packed=packed)
                      for i in range(0, B, lim)]
             return {k: torch.cat([p[k] for p in parts]) for k in parts[0]}
         lib = _lib.load()
         st = _lib.stream_handle(dev)
         pb = self._prep_buffers(B, N, dev)
         self._prep_csr_rows(pb, 0, B, N, (node_feats, node_qr, nbr, row_offsets), row0, st)
-        return self._trunk(pb, B, N, dev, request_moves_left)
+        return self._trunk(pb, B, N, dev, request_moves_left, packed)
 
     # ---- graph-captured serve forward (the reference's _GraphCache,
     # inference.py:226-352): one captured trunk per (batch bucket, Npad,
@@ -608,12 +647,13 @@ class HipForward:
             )
         return self._trunk(pb, B, N, dev, request_moves_left)
 
-    def _trunk(self, pb: SimpleNamespace, B: int, N: int, dev, request_moves_left: bool) -> dict:
+    def _trunk(self, pb: SimpleNamespace, B: int, N: int, dev, request_moves_left: bool,
+               packed=None) -> dict:
         """Everything after the input preparation: stem, blocks, tail, heads."""
 
         if self.fp32:
-            return self._trunk32(pb, B, N, dev, request_moves_left)
-        P = self.weights(dev)
+            return self._trunk32(pb, B, N, dev, request_moves_left, packed)
+        P = self.weights(dev) if packed is None else packed
         C, H, d, dpad = P.C, P.H, P.d, P.dpad
         S = N + NUM_TOKENS
         lib = _lib.load()
@@ -621,6 +661,8 @@ class HipForward:
         bf = torch.bfloat16
         idx, mask8, coords32 = pb.idx, pb.mask8, pb.coords32
         seq_lens, seq_mask, xin = pb.seq_lens, pb.seq_mask, pb.xin
+        if B > 0 and not self.keep_buffers and self.timeline is None and not self.use_fused_attn:
+            return self._trunk_native(P, pb, B, N, dev, request_moves_left, lib, st)
         seq = torch.empty((B, S, C), dtype=bf, device=dev)
         # the token rows' residual stream is seq (bf16) + tok_lo (bf16): the
         # rounding remainder of every update, kept by the residual kernels
@@ -826,11 +868,53 @@ class HipForward:
             )
         return out
 
-    def _trunk32(self, pb: SimpleNamespace, B: int, N: int, dev, request_moves_left: bool) -> dict:
+    def _trunk_native(self, P, pb, B, N, dev, request_moves_left, lib, st) -> dict:
+        """_trunk's launches from one native call (shrimp_forward), the same
+        kernels by the same rules on one workspace: the host builds no argument
+        list per launch (12 blocks: 0.5 ms of Python, 40 us here)."""
+
+        C, H, d, dpad = P.C, P.H, P.d, P.dpad
+        S = N + NUM_TOKENS
+        fused_qkv = P.fused_qkv and self.use_fused_qkv
+        staged = (fused_qkv and self.use_staged_attn and self.use_linear_bias and C == 128
+                  and d == dpad and attn_staged_supported(H, S, dpad))
+        big = self._fused_batch(B, N, dev)
+        block = self.use_fused_block and big and conv_block_supported(7, N, C, C)
+        pair = block and self.use_block_pair and conv_block_pair_supported(7, N, C, C)
+        tail = self.use_fused_tail and big and bool(lib.shrimp_policy_tail_supported(N, C))
+        flags = sum(bit for bit, on in (
+            (_lib.FWD_STAGED, staged), (_lib.FWD_QKV, fused_qkv),
+            (_lib.FWD_MLP, P.fused_mlp and self.use_fused_mlp), (_lib.FWD_BLOCK, block),
+            (_lib.FWD_PAIR, pair), (_lib.FWD_TAIL, tail),
+            (_lib.FWD_LINEAR_BIAS, self.use_linear_bias)) if on)
+        # padded channels that no kernel writes are zeros of the caller's
+        qkv = None
+        if not staged and d != dpad and not (fused_qkv and C in (96, 192)):
+            qkv = torch.zeros((3, B, H, S, dpad), dtype=torch.bfloat16, device=dev)
+        net = self._net_words(P)
+        nbytes = lib.shrimp_forward_bytes(net, B, N, flags, qkv is None)
+        if nbytes <= 0:
+            raise ValueError(f"forward: bad shape (B={B}, N={N}, C={C}, H={H})")
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        value = torch.empty((B, VALUE_BINS), dtype=torch.float32, device=dev)
+        ml = torch.empty_like(value) if request_moves_left else None
+        policy = torch.empty((B, N), dtype=torch.float32, device=dev)
+        io = _lib.words(
+            pb.idx.data_ptr(), pb.mask8.data_ptr(), pb.coords32.data_ptr(), pb.seq_lens.data_ptr(),
+            pb.seq_mask.data_ptr(), pb.xin.data_ptr(), ws.data_ptr(), _lib.ptr(qkv) or 0,
+            policy.data_ptr(), value.data_ptr(), _lib.ptr(ml) or 0, B, N, flags)
+        _lib.check(lib.shrimp_forward(net, io, st), "forward")
+        out = {"policy": policy, "value": value}
+        if request_moves_left:
+            out["moves_left"] = ml
+        return out
+
+    def _trunk32(self, pb: SimpleNamespace, B: int, N: int, dev, request_moves_left: bool,
+                 packed=None) -> dict:
         """The fp32 serve mode's trunk: the launch sequence of _trunk on the fp32
         kernels (model.py:395-514, 905-1020), fp32 activations throughout."""
 
-        P = self.weights(dev)
+        P = self.weights(dev) if packed is None else packed
         C, H, d = P.C, P.H, P.d
         S = N + NUM_TOKENS
         lib = _lib.load()

@@ -113,6 +113,16 @@ int shrimp_pack_linear_weight(const float* w, void* packed, int in_features, int
  * dst is 16-byte aligned. */
 int shrimp_op_prep(const int64_t* jobs, int n_jobs, void* stream);
 
+/* The bf16 trunk of one forward, stem to heads (model.py:395-514, 865,
+ * 905-1020), as the launch sequence of the entry points below on prepared inputs
+ * (shrimp_prep_inputs / shrimp_prep_csr). `net` and `io` are int64 words in host
+ * memory, read before the call returns (word order: csrc/forward.cpp): the packed
+ * weights' addresses, and the call's buffers, sizes and kernel choices.
+ * shrimp_forward_bytes gives the workspace (256-byte aligned) of a call, 0 for a
+ * bad shape; own_qkv 0 when the caller passes its own q / k / v planes. */
+int64_t shrimp_forward_bytes(const int64_t* net, int B, int N, int flags, int own_qkv);
+int shrimp_forward(const int64_t* net, const int64_t* io, void* stream);
+
 /* ------------------------------------------------------------------------
  * Gather-GEMM hex / ray-tap convolution with fused epilogue.
  *

@@ -777,3 +777,35 @@ def test_evaluator_keeps_its_packed_weights():
     payload, _ = synthetic.serve_payload("cfg4_spec", 10)
     ShrimpEvaluator(net, "cuda").evaluate_payload(payload)
     assert rt._packed is packed
+
+
+# the native launch sequence against the Python one (which a timeline selects):
+# padded q / k / v channels the caller zeroes (32 channels), the weight-streamed
+# widths, 128 channels on both sides of the fused kernels' batch, and every
+# kernel choice that changes the sequence
+@pytest.mark.parametrize("c,h,layout,batch", [
+    (32, 4, "CCA", 5), (96, 4, "CCCACA", 9), (128, 8, "CCACA", 3), (128, 8, "CCACA", 140),
+    (192, 3, "CAA", 4),
+])
+def test_native_sequence_matches_python(c, h, layout, batch):
+    from shrimp import synthetic
+
+    net = _net(c, h, layout, seed=5, mode="heads")
+    rt = net.hip_runtime()
+    b = synthetic.position_batch("cfg0", 5, seed=9)
+    args = [torch.cat([b[k]] * -(-batch // 5))[:batch].to(DEV) for k in ("feats", "nbr", "mask", "coords")]
+    toggles = ("use_fused_block", "use_block_pair", "use_fused_tail", "use_fused_mlp", "use_fused_qkv",
+               "use_staged_attn", "use_linear_bias")
+    for off in (None, *toggles):
+        if off:
+            setattr(rt, off, False)
+        got = net.forward_policy_value(*args, request_moves_left=True)
+        rt.timeline = []
+        want = net.forward_policy_value(*args, request_moves_left=True)
+        assert len(rt.timeline) > 4
+        rt.timeline = None
+        if off:
+            setattr(rt, off, True)
+        assert set(got) == set(want)
+        for k in want:
+            assert torch.equal(got[k], want[k]), (off, k)

@@ -36,7 +36,7 @@
 // the SIMD cycles together, the rest the chain of one chunk. Measured on MI355X:
 // 111 positions, S = 584, H = 3, D = 64 1873 us (one query row per thread) -> 80 us;
 // 150 positions, S = 328, H = 4, D = 32 67 -> 41 us; the pair tensor at 60
-// positions, S = 341, H = 3, D = 64 94 -> 25.5 us. Two 32-key steps per chunk as a
+// positions, S = 341, H = 3, D = 64 94 -> 23 us. Two 32-key steps per chunk as a
 // rolled loop keep 139 VGPRs (unrolled 168 with 49 spilled).
 #include <type_traits>
 
@@ -61,21 +61,53 @@ constexpr float LAZY_MAX = 8.0f; // scores above m + this move the offset
 
 typedef __attribute__((address_space(3))) void lds_dst_t;
 typedef __attribute__((address_space(3))) const unsigned char lds_cu8;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 SHRIMP_DEV int clampi(int x, int m) { return min(max(x, -m), m); }
 
-// LDS byte addresses as plain integers (no base pointer added per read).
+// LDS byte addresses as plain integers: no base pointer added per read, and
+// the compiler, which takes a read through a pointer into the workgroup's LDS
+// to alias the chunk DMA in flight and waits for it (vmcnt 0), leaves the
+// ordering to the wait and barrier that end each chunk (82.8 -> 81.2 us at
+// D = 64, S = 584, 13.2 -> 12.8 us for a dozen positions at D = 32).
 SHRIMP_DEV int lds_addr(const void* p) { return (int)(uintptr_t)(lds_cu8*)p; }
+SHRIMP_DEV unsigned lds_u32(int addr) {
+  return *(__attribute__((address_space(3))) const unsigned*)(uintptr_t)(unsigned)addr;
+}
+SHRIMP_DEV unsigned lds_u8(int addr) {
+  return *(__attribute__((address_space(3))) const unsigned char*)(uintptr_t)(unsigned)addr;
+}
 SHRIMP_DEV float lds_f32(int addr) {
   return *(__attribute__((address_space(3))) const float*)(uintptr_t)(unsigned)addr;
 }
 SHRIMP_DEV u32x4 lds_16(int addr) {
   return *(__attribute__((address_space(3))) const u32x4*)(uintptr_t)(unsigned)addr;
 }
-SHRIMP_DEV u32x2 lds_tr(int addr) {
-  return __builtin_bit_cast(
-      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(unsigned)addr));
+// V^T fragments of 32 keys: for each address a pair of transposing reads, RB16
+// bytes (16 keys) apart. In assembly with its own wait: the builtin is taken to
+// alias the next chunk's DMA, and the compiler waits for that before the first
+// read of every chunk.
+template <int RB16>
+SHRIMP_DEV void lds_tr(const int (&at)[4], u32x2 (&a)[4], u32x2 (&b)[4]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %4, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %1, %9\n\tds_read_b64_tr_b16 %5, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %2, %10\n\tds_read_b64_tr_b16 %6, %10 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %3, %11\n\tds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]),
+        "=&v"(b[3])
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(RB16)
+      : "memory");
+}
+template <int RB16>
+SHRIMP_DEV void lds_tr(const int (&at)[2], u32x2 (&a)[2], u32x2 (&b)[2]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %2, %4 offset:%6\n\t"
+      "ds_read_b64_tr_b16 %1, %5\n\tds_read_b64_tr_b16 %3, %5 offset:%6\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(b[0]), "=&v"(b[1])
+      : "v"(at[0]), "v"(at[1]), "n"(RB16)
+      : "memory");
 }
 
 // Swizzle of row r's 16-byte pieces (D / 8 per row): a 128-byte line of LDS
@@ -97,11 +129,11 @@ struct StreamQuery {
   bool qtok[QB];
 };
 
-struct StreamLds {
-  const int* kkey;        // LINEAR: LDS address of the key's table row for offset code 0
-  const int2* kqr;        // CLAMP: coordinates
-  const unsigned char* kcls;
-  const float* tab;       // CLAMP and PAIR tables
+struct StreamLds {      // LDS byte addresses
+  int keys;             // LINEAR: per key the address of its table row for offset code 0;
+                        // CLAMP: its coordinates
+  int kcls;             // key classes, one byte each
+  int tab;              // CLAMP and PAIR tables
   float tokb[3];          // (cell query, token key), (token query, cell key), (token, token)
   float inv_scale;
   int npos;
@@ -137,16 +169,16 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
 #pragma unroll
   for (int kb = 0; kb < NKB; ++kb) {
     const int key0 = k0 + kb * 16 + lg * 4;
-    int4 kk{0, 0, 0, 0}, kr{0, 0, 0, 0};
+    u32x4 kk{0, 0, 0, 0}, kr{0, 0, 0, 0};
     if constexpr (PATH == PATH_LINEAR) {
-      kk = *reinterpret_cast<const int4*>(s.kkey + key0);
+      kk = lds_16(s.keys + key0 * 4);
     } else if constexpr (PATH == PATH_CLAMP) {
-      const int4 a0 = *reinterpret_cast<const int4*>(s.kqr + key0);
-      const int4 a1 = *reinterpret_cast<const int4*>(s.kqr + key0 + 2);
-      kk = int4{a0.x, a0.z, a1.x, a1.z};
-      kr = int4{a0.y, a0.w, a1.y, a1.w};
+      const u32x4 a0 = lds_16(s.keys + key0 * 8), a1 = lds_16(s.keys + key0 * 8 + 16);
+      kk = u32x4{a0[0], a0[2], a1[0], a1[2]};
+      kr = u32x4{a0[1], a0[3], a1[1], a1[3]};
     }
-    const int kv[4] = {kk.x, kk.y, kk.z, kk.w}, rv[4] = {kr.x, kr.y, kr.z, kr.w};
+    const int kv[4] = {(int)kk[0], (int)kk[1], (int)kk[2], (int)kk[3]};
+    const int rv[4] = {(int)kr[0], (int)kr[1], (int)kr[2], (int)kr[3]};
     float bias[QB][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -156,15 +188,16 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
           bias[qb][j] = lds_f32(kv[j] - w.qkey[qb]);
         } else if constexpr (PATH == PATH_CLAMP) {
           const int M = a.lut_m, W = 2 * M + 1;
-          bias[qb][j] = s.tab[(clampi(kv[j] - w.qq[qb], M) + M) * W + clampi(rv[j] - w.qr[qb], M) + M];
+          bias[qb][j] = lds_f32(
+              s.tab + ((clampi(kv[j] - w.qq[qb], M) + M) * W + clampi(rv[j] - w.qr[qb], M) + M) * 4);
         } else {
           const int p = (int)((pd[qb][kb] >> (8 * j)) & 0xFF);
-          bias[qb][j] = s.tab[min(p, s.npos - 1)];
+          bias[qb][j] = lds_f32(s.tab + min(p, s.npos - 1) * 4);
         }
       }
     if ((special >> kb) & 1) {
       unsigned cls = 0;
-      if constexpr (PATH != PATH_PAIR) cls = *reinterpret_cast<const unsigned*>(s.kcls + key0);
+      if constexpr (PATH != PATH_PAIR) cls = lds_u32(s.kcls + key0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int c = (cls >> (8 * j)) & 0xFF;
@@ -244,14 +277,18 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
       pp[qb] = u32x4{pf[qb][kp].x, pf[qb][kp].y, pf[qb][kp + 1].x, pf[qb][kp + 1].y};
       w.l[qb] = mfma16x16x32(u32x4{one2, one2, one2, one2}, pp[qb], w.l[qb]);
     }
+    int at[KD];
+    u32x2 v0[KD], v1[KD];
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd) {
-      const int at = vlane + kp * 16 * RB + (((kd * 2 + ((lr & 3) >> 1)) ^ vsw) << 4);
-      const u32x2 v0 = lds_tr(at), v1 = lds_tr(at + 16 * RB);
+    for (int kd = 0; kd < KD; ++kd)
+      at[kd] = vlane + kp * 16 * RB + (((kd * 2 + ((lr & 3) >> 1)) ^ vsw) << 4);
+    lds_tr<16 * RB>(at, v0, v1);
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb)
-        w.o[qb][kd] = mfma16x16x32(u32x4{v0.x, v0.y, v1.x, v1.y}, pp[qb], w.o[qb][kd]);
-    }
+        w.o[qb][kd] =
+            mfma16x16x32(u32x4{v0[kd].x, v0[kd].y, v1[kd].x, v1[kd].y}, pp[qb], w.o[qb][kd]);
   }
 }
 
@@ -353,7 +390,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
       const int row = (j - tensor * PPR) * (64 / PPR) + lane / PPR;
       const int piece = (lane % PPR) ^ swz<D>(row);
       const int key = c * KC + row;
-      const bool ok = PAIR ? key < L : kcls[key] != KEY_DEAD;
+      const bool ok = PAIR ? key < L : lds_u8(lds_addr(kcls) + key) != KEY_DEAD;
       const uint32_t off =
           ok ? (uint32_t)((base + (int64_t)key * D + piece * 8) * 2) : SHRIMP_OOB_OFFSET;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tensor ? vrs : krs,
@@ -362,10 +399,9 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
     }
   };
   StreamLds s;
-  s.kkey = kkey;
-  s.kqr = kqr;
-  s.kcls = kcls;
-  s.tab = reinterpret_cast<const float*>(tabs);
+  s.keys = lds_addr(kqr);
+  s.kcls = lds_addr(kcls);
+  s.tab = lds_addr(tabs);
   s.npos = npos;
   s.inv_scale = 1.0f / scale;
   bool linear = false;
@@ -490,8 +526,11 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
         unsigned x = 0;
         if (c * KC + KC <= S) {
           __builtin_memcpy(&x, row + key, 4);
+        } else if (S >= 4) {  // past the row's end: its last four keys, shifted
+          const int at = min(key, S - 4);
+          __builtin_memcpy(&x, row + at, 4);
+          x = key - at < 4 ? x >> (8 * (key - at)) : 0u;
         } else {
-#pragma unroll
           for (int j = 0; j < 4; ++j)
             if (key + j < S) x |= (unsigned)row[key + j] << (8 * j);
         }
@@ -535,7 +574,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
           const int over = L - c * KC;  // keys of the chunk inside the bound
           special = over >= KC ? 0 : (15 << (over >> 4)) & 15;
         } else {
-          special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)flags[c]);
+          special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)lds_u8(lds_addr(flags) + c));
         }
 #pragma unroll 1
         for (int kb = 0; kb < 4 && c * KC + kb * 16 < L; kb += NKB) {

@@ -155,6 +155,7 @@ def pack_raytap_weight(weight: torch.Tensor) -> torch.Tensor:
 def _packed_weight(weight: torch.Tensor) -> torch.Tensor:
     """pack_raytap_weight, an fp32 weight rounded and packed in one launch."""
 
+    require_device(weight, "pack_raytap_weight")
     t, c, cout = weight.shape
     nbytes = _load().shrimp_raytap_wpack_bytes(c, cout)
     if weight.dtype != torch.float32 or t != 7 or nbytes == 0:
@@ -278,9 +279,9 @@ def hex_conv_ln_raytap(
     cout = weight.shape[-1]
     xh = _fp16_view(x)
     gi = gather_idx
-    if gi.dtype == torch.int64:
+    if gi.dtype == torch.int64 and gi.stride(1) > 0 and max(gi.stride()) < 1 << 30:
         # only slot 0 is read: the low dwords of the int64 indices in place
-        gi = (gi if gi.stride(-1) == 1 else gi.contiguous()).view(torch.int32)
+        gi = gi[..., 0].unsqueeze(-1).view(torch.int32)
     else:
         gi = gi.to(torch.int32)
         if gi.stride(-1) != 1:

@@ -430,6 +430,7 @@ def prep_rows(t: torch.Tensor, pad: int, jobs: list) -> torch.Tensor:
     """t (..., C) as contiguous bf16 rows of ``pad`` channels (zeros past C): t
     itself, or a tensor that a job of ``jobs`` (_lib.op_prep) fills."""
 
+    require_device(t, "operand rows")
     c = t.shape[-1]
     if t.dtype == torch.bfloat16 and c == pad and t.is_contiguous():
         return t
@@ -446,6 +447,7 @@ def prep_rows(t: torch.Tensor, pad: int, jobs: list) -> torch.Tensor:
 def prep_index(t: torch.Tensor, jobs: list) -> torch.Tensor:
     """t as contiguous int32: t itself, or a tensor that a job fills (int64)."""
 
+    require_device(t, "operand indices")
     if t.dtype != torch.int64:
         return t.to(torch.int32).contiguous()
     t = t.contiguous()
@@ -464,6 +466,7 @@ def mask_bytes(mask: torch.Tensor) -> torch.Tensor:
 
 def _conv_common(x, gather_idx, mask, weight, bias, ln_weight, ln_bias, eps, relu):
     require_device(x, "shrimp::hex_conv")
+    require_device(weight, "shrimp::hex_conv weight")
     b, n, c = x.shape
     t, cin, cout = weight.shape
     cp = cin_pad_of(c)

@@ -213,7 +213,7 @@ class HipForward:
                 if p is not None:
                     key.append(p.data_ptr())
                     key.append(p._version)
-            todo.extend(m._modules.values())
+            todo.extend(c for c in m._modules.values() if c is not None)
         return tuple(key)
 
     @property

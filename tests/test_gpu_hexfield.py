@@ -268,3 +268,31 @@ def test_conv_ln_raytap_bench_shape_samples():
         torch.testing.assert_close(got[sel].double().cpu(), want, atol=5e-3, rtol=0)
     assert not torch.isnan(got).any()
     assert math.isfinite(float(got.float().abs().max()))
+
+
+def test_conv_ln_raytap_int64_index_forms():
+    """int64 gather indices are read in place where their layout allows it: a
+    column slice, a one-slot view whose last stride is not 1, a view of rows
+    that all share one index (copied first), int32 beside them."""
+
+    from hexfield_eq import build_ray_gather_index, build_tap_reach, hex_conv_ln_raytap
+
+    coords, mask = _batch(["disk4", "chain"], 70, seed=31)
+    x, w, bias, lnw, lnb, alpha, raylen, _ = (t.to(DEV) if torch.is_tensor(t) else t
+                                              for t in _k1_inputs(coords, mask, 96, 96, 32))
+    b, n = mask.shape
+    m = torch.from_numpy(mask).to(DEV)
+    ray = build_ray_gather_index(torch.from_numpy(coords).to(DEV), m)
+    reach = build_tap_reach(raylen)
+    gidx = torch.from_numpy(tables.gather_index(_nbr(coords, mask))).to(DEV).long()
+
+    def run(g):
+        return hex_conv_ln_raytap(x, g, m, w, bias, lnw, lnb, ray, reach, alpha, 1e-5, True, 8)
+
+    want = run(gidx.int())
+    wide = torch.cat([gidx, gidx], dim=-1)
+    by_slot = gidx.permute(2, 0, 1).contiguous().permute(1, 2, 0)
+    for g in (gidx, wide[..., :7], gidx[..., :1], by_slot, by_slot[..., :1]):
+        assert torch.equal(run(g), want), (tuple(g.shape), g.stride())
+    shared = gidx[:, 3:4].expand(b, n, 7)
+    assert torch.equal(run(shared), run(shared.int().contiguous()))

@@ -1464,3 +1464,22 @@ def test_op_prep_matches_torch():
                 (w.data_ptr(), w.data_ptr(), 0, 1, 4, 8, 12, 0)):
         with pytest.raises(RuntimeError, match="op_prep"):
             _lib.op_prep([bad], st)
+
+
+# operands that only a device kernel reads now are refused on the host, as the
+# library conversions before them refused them
+def test_operator_operands_stay_checked():
+    from hexfield_eq import ops as hops
+    from shrimp import ops
+
+    with pytest.raises(RuntimeError, match="ROCm device"):
+        ops.prep_rows(torch.zeros(4, 32), 32, [])
+    with pytest.raises(RuntimeError, match="ROCm device"):
+        ops.prep_index(torch.zeros(4, dtype=torch.int64), [])
+    with pytest.raises(RuntimeError, match="ROCm device"):
+        hops._packed_weight(torch.zeros(7, 64, 64))
+    x, m = torch.zeros(1, 4, 32, device=DEV), torch.ones(1, 4, dtype=torch.bool, device=DEV)
+    g = torch.zeros(1, 4, 7, dtype=torch.int64, device=DEV)
+    with pytest.raises(RuntimeError, match="ROCm device"):
+        ops._conv_common(x, g, m, torch.zeros(7, 32, 32), torch.zeros(32, device=DEV), None, None, 1e-5,
+                         False)

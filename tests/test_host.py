@@ -275,3 +275,22 @@ def test_busy_trace_report_arithmetic():
     assert rep["mean_batch"] == 20.0 and rep["median_batch"] == 20.0
     assert rep["mean_forward_ms"] == 4.0 and rep["median_forward_ms"] == 4.0
     assert rep["mean_ms_per_state"] == 0.2
+
+
+def test_parameter_key_walks_every_module():
+    """The key of the packed weights sees every parameter, a submodule
+    registered as None included."""
+
+    from shrimp.model import ShrimpNet
+
+    net = ShrimpNet(channels=32, attention_heads=4, trunk_layout="CA")
+    rt, dev = net.hip_runtime(), torch.device("cuda", 0)
+    net.register_module("absent", None)
+    key = rt._param_key(dev)
+    assert {p.data_ptr() for p in net.parameters()} <= set(key)
+    for p in net.parameters():
+        before = rt._param_key(dev)
+        with torch.no_grad():
+            p.add_(0)
+        assert rt._param_key(dev) != before
+    assert rt._param_key(dev) != key and rt._param_key(torch.device("cuda", 1)) != rt._param_key(dev)

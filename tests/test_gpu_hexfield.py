@@ -181,6 +181,35 @@ def test_ray_attn_bench_shape_samples_and_variants_agree():
         torch.testing.assert_close(staged[sel].double().cpu(), want, atol=3e-3, rtol=0)
 
 
+# the staged kernel against the global one and the oracle: rows around a wave's
+# DMA and a workgroup's pass, one head left over, LDS past 64 KiB, slots pointing
+# past seq_lens (not staged), and a NaN row that no slot names
+@pytest.mark.parametrize("n,h,d", [(1, 6, 16), (31, 5, 16), (32, 6, 32), (129, 3, 64), (257, 6, 16),
+                                   (505, 7, 16), (250, 6, 32)])
+def test_ray_attn_staged_rows(n, h, d):
+    from hexfield_eq import ray_attn
+    from hexfield_eq.ops import ray_attn_variant
+
+    b, gen = 5, torch.Generator().manual_seed(n + h + d)
+    (q, k, v), sb, rl = _ray_inputs(b, h, n, d, n)
+    idx = torch.randint(0, n + 1, (b, n, 32), generator=gen, dtype=torch.int32)
+    idx[:, :, 0] = torch.arange(n)
+    sl = torch.tensor([n, max(n - 1, 1), (n + 1) // 2, 1, 0], dtype=torch.int32)
+    if n > 2:
+        idx[0] = torch.where(idx[0] == 2, n, idx[0])  # position 0 never reads row 2
+        k[0, :, 2] = v[0, :, 2] = float("nan")
+    args = (q, k, v, idx.to(DEV), sb.to(DEV), rl.to(DEV), sl.to(DEV), True)
+    got = ray_attn(*args)
+    prev = ray_attn_variant(1)
+    try:
+        assert torch.equal(got, ray_attn(*args))
+    finally:
+        ray_attn_variant(prev)
+    z = lambda t: t.cpu().nan_to_num(0.0)
+    want = ohf.ray_attn(q.cpu(), z(k), z(v), idx, sb, rl, sl, True)
+    torch.testing.assert_close(got.double().cpu(), want, atol=3e-3, rtol=0)
+
+
 # ---- K1 ---------------------------------------------------------------------------------
 
 
@@ -277,7 +306,7 @@ def test_conv_ln_raytap_int64_index_forms():
 
     from hexfield_eq import build_ray_gather_index, build_tap_reach, hex_conv_ln_raytap
 
-    coords, mask = _batch(["disk4", "chain"], 70, seed=31)
+    coords, mask = _batch(["disk4", "disk3"], 70, seed=31)
     x, w, bias, lnw, lnb, alpha, raylen, _ = (t.to(DEV) if torch.is_tensor(t) else t
                                               for t in _k1_inputs(coords, mask, 96, 96, 32))
     b, n = mask.shape

@@ -357,9 +357,8 @@ __global__ __launch_bounds__(RA_THREADS) void ray_attn_kernel(const shrimp_ray_a
 
 // ---- ray-tap conv + LayerNorm (K1) -------------------------------------------------
 
-constexpr int RT_MB = 4;  // 16-row blocks per wave (64 rows)
 constexpr int RT_MAX_N = 512;
-constexpr int RT_MAX_WAVES = RT_MAX_N / (16 * RT_MB);
+constexpr int RT_HALF_N = 384;  // most rows of 32-row waves (three per SIMD)
 
 // Slot of step k = 1 for direction tap t = 1..6 (DIRECTIONS (1,0) (0,1) (-1,1)
 // (-1,0) (0,-1) (1,-1) against the axes Q (1,0), R (0,1), QR (1,-1)):
@@ -369,10 +368,10 @@ __constant__ int RT_SLOT_BASE[6] = {1, 11, 26, 6, 16, 21};
 __host__ __device__ constexpr int rt_row_stride(int cin) { return cin * 2 + 16; }
 __host__ __device__ constexpr int rt_out_stride(int cout) { return cout * 2 + 16; }
 // Bytes of the row region: the x rows (N + 1 of them) during the taps, the
-// output rows (64 per wave) in the epilogue.
-__host__ __device__ inline uint32_t rt_rows_bytes(int N, int cin, int cout, int waves) {
+// output rows (`rows`: whole waves) in the epilogue.
+__host__ __device__ inline uint32_t rt_rows_bytes(int N, int cin, int cout, int rows) {
   const uint32_t xr = (uint32_t)(N + 1) * rt_row_stride(cin);
-  const uint32_t orr = (uint32_t)waves * 64 * rt_out_stride(cout);
+  const uint32_t orr = (uint32_t)rows * rt_out_stride(cout);
   return xr > orr ? xr : orr;
 }
 
@@ -404,10 +403,14 @@ SHRIMP_DEV f32x4 mfma_f16(u32x4 a, u32x4 b, f32x4 c) {
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-template <int CIN, int COUT>
-__global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
+// MB blocks of 16 rows per wave. The chain of one wave bounds a launch while a
+// compute unit holds few of them, and 32-row waves (MB = 2) are twice as many and
+// half as long, at twice the weight reads. Same products in the same order, so
+// the same bits.
+template <int CIN, int COUT, int MB>
+__global__ __launch_bounds__(MB == 4 ? RT_MAX_N : 2 * RT_HALF_N) void conv_ln_raytap_kernel(
     const shrimp_raytap_args a) {
-  constexpr int KC = CIN / 32, NB = COUT / 16, MB = RT_MB;
+  constexpr int KC = CIN / 32, NB = COUT / 16, WR = 16 * MB;  // rows per wave
   constexpr int RS = rt_row_stride(CIN);
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int N = a.N;
@@ -415,7 +418,7 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
   const int lane = (int)threadIdx.x & 63, wave = wave_id();
   const int lr = lane & 15, lg = lane >> 4;
   unsigned char* xs = lds;  // (N + 1) rows of RS bytes, later the output rows
-  unsigned char* al = lds + rt_rows_bytes(N, CIN, COUT, (int)(blockDim.x >> 6));  // alpha (5, CIN) fp16
+  unsigned char* al = lds + rt_rows_bytes(N, CIN, COUT, (int)(blockDim.x >> 6) * WR);  // alpha (5, CIN) fp16
 
   // Stage the position's rows, the zero row N and alpha.
   {
@@ -432,12 +435,12 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
           *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(a.alpha) + c * 16);
   }
 
-  // This lane's rows: wave * 64 + mb * 16 + lr.
+  // This lane's rows: wave * WR + mb * 16 + lr.
   int rn[MB];
   bool rv[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    rn[mb] = wave * 64 + mb * 16 + lr;
+    rn[mb] = wave * WR + mb * 16 + lr;
     rv[mb] = rn[mb] < N;
   }
   const int32_t* rib = a.ray_idx + (int64_t)b * a.r_sb;
@@ -475,9 +478,9 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
       if ((c % a.corb) >= (a.corb >> 1)) sidebits |= 1u << (2 * kc + h);
     }
 
-  // Ray rows and reach of one direction tap for row wave * 64 + lane, loaded
+  // Ray rows and reach of one direction tap for row wave * WR + lane, loaded
   // one tap ahead so the global latency hides behind the previous tap.
-  const int trow = wave * 64 + lane;
+  const int trow = lane < WR ? wave * WR + lane : N;
   int pj[RAY_STEPS];
   uint32_t preach = 0;
   auto tap_fetch = [&](int t) {
@@ -523,12 +526,12 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
     for (int nb = 0; nb < NB; ++nb) w[nb] = wl[nb];
   }
 
-  // Taps 1..6. Per tap, lane l of each wave writes, for row wave * 64 + l, the
+  // Taps 1..6. Per tap, lane l of each wave writes, for row wave * WR + l, the
   // visible row of every step and side into the wave's slice of `vt` (5 dwords,
   // own | opp << 16, N = the zero row; 8 dwords per row); every chunk of the tap
   // reads it back for its rows. The slice belongs to one wave and a wave's LDS
   // accesses complete in issue order, so no workgroup barrier is needed.
-  uint32_t* vt = reinterpret_cast<uint32_t*>(al + RAY_STEPS * CIN * 2) + wave * 64 * 8;
+  uint32_t* vt = reinterpret_cast<uint32_t*>(al + RAY_STEPS * CIN * 2) + wave * WR * 8;
   for (int t = 0; t < 6; ++t) {
     {
       const int r0 = (int)(preach & 0xFF), r1 = (int)(preach >> 8);
@@ -540,8 +543,10 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
         const uint32_t opp = pres && k + 1 <= r1 ? (uint32_t)pj[k] : (uint32_t)N;
         vr[k] = own | (opp << 16);
       }
-      *reinterpret_cast<u32x4*>(vt + lane * 8) = u32x4{vr[0], vr[1], vr[2], vr[3]};
-      vt[lane * 8 + 4] = vr[4];
+      if (lane < WR) {
+        *reinterpret_cast<u32x4*>(vt + lane * 8) = u32x4{vr[0], vr[1], vr[2], vr[3]};
+        vt[lane * 8 + 4] = vr[4];
+      }
     }
     if (t + 1 < 6) tap_fetch(t + 1);
     __builtin_amdgcn_wave_barrier();
@@ -634,12 +639,12 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
     rstd[mb] = rsqrtf(sum_groups_swap(q) * (1.0f / COUT) + a.eps);
     live[mb] = rv[mb] && mk[rn[mb]] != 0;
   }
-  // The output rows go through LDS (each wave's 64 rows in its own slice over
+  // The output rows go through LDS (each wave's rows in its own slice over
   // the x rows, which every wave has finished reading) and leave as whole
   // 16-byte row pieces: 8-byte stores per lane would write 32-byte segments.
   __syncthreads();
   constexpr int OS = rt_out_stride(COUT);
-  unsigned char* ob = xs + (size_t)wave * 64 * OS;
+  unsigned char* ob = xs + (size_t)wave * WR * OS;
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     const int c0 = nb * 16 + lg * 4;
@@ -664,9 +669,9 @@ __global__ __launch_bounds__(64 * RT_MAX_WAVES) void conv_ln_raytap_kernel(
   constexpr int CPR = COUT / 8;  // 16-byte pieces per output row
   const int ch = lane & 15;
 #pragma unroll
-  for (int it = 0; it < 16; ++it) {
+  for (int it = 0; it < WR / 4; ++it) {
     const int r = it * 4 + (lane >> 4);
-    const int row = wave * 64 + r;
+    const int row = wave * WR + r;
     if (ch < CPR && row < N) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(ob + r * OS + ch * 16);
       *reinterpret_cast<u32x4*>(a.out + (int64_t)b * a.o_sb + (int64_t)row * a.o_sn + ch * 8) = v;
@@ -689,16 +694,35 @@ int launch_ray_attn(const shrimp_ray_attn_args& a, bool stage, hipStream_t st) {
   return check_launch("ray_attn");
 }
 
-template <int CIN>
-int launch_raytap_cin(const shrimp_raytap_args& a, size_t lds, hipStream_t st) {
-  const int waves = (a.N + 16 * RT_MB - 1) / (16 * RT_MB);
+template <int CIN, int COUT>
+int launch_raytap(const shrimp_raytap_args& a, hipStream_t st) {
+  // 64-row waves where those fill a compute unit already (two workgroups of three
+  // or four waves at 242-256 VGPRs; 32-row waves at 128 VGPRs, Cout = 64, fit four
+  // per SIMD and win there too) and past the 32-row waves' 384 rows. Measured, 64
+  // against 32 rows, C = Cout: 96 channels B = 200, N = 300 38.9 / 30.3 us; B = 512,
+  // N = 300 78.5 / 62.4; B = 256, N = 256 31.1 / 25.0, B = 260 39.6 / 44.4; B = 1024,
+  // N = 256 83.9 / 95.1, N = 128 47.4 / 46.9, N = 64 32.4 / 26.4. 128 channels
+  // B = 8, N = 256 35.7 / 29.0; B = 1024, N = 256 112.1 / 128.9. 64 channels
+  // B = 1024, N = 256 55.9 / 55.0.
+  const bool full = COUT > 64 && a.N > 128 && a.N <= 256 && a.B > cu_count();
+  const int mb = full || a.N > RT_HALF_N ? 4 : 2;
+  const int waves = (a.N + 16 * mb - 1) / (16 * mb);
+  const size_t lds = (size_t)rt_rows_bytes(a.N, CIN, COUT, waves * 16 * mb) +
+                     (size_t)RAY_STEPS * CIN * 2 + (size_t)waves * 16 * mb * 8 * 4;
+  SHRIMP_REQUIRE(lds <= (size_t)max_lds_per_block(), "conv_ln_raytap: needs %zu bytes of LDS", lds);
   const dim3 grid((unsigned)a.B), block((unsigned)(64 * waves));
-  switch (a.Cout) {
-    case 64: hipLaunchKernelGGL((conv_ln_raytap_kernel<CIN, 64>), grid, block, lds, st, a); break;
-    case 96: hipLaunchKernelGGL((conv_ln_raytap_kernel<CIN, 96>), grid, block, lds, st, a); break;
-    default: hipLaunchKernelGGL((conv_ln_raytap_kernel<CIN, 128>), grid, block, lds, st, a); break;
-  }
+  if (mb == 4) hipLaunchKernelGGL((conv_ln_raytap_kernel<CIN, COUT, 4>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((conv_ln_raytap_kernel<CIN, COUT, 2>), grid, block, lds, st, a);
   return check_launch("conv_ln_raytap");
+}
+
+template <int CIN>
+int launch_raytap_cin(const shrimp_raytap_args& a, hipStream_t st) {
+  switch (a.Cout) {
+    case 64: return launch_raytap<CIN, 64>(a, st);
+    case 96: return launch_raytap<CIN, 96>(a, st);
+    default: return launch_raytap<CIN, 128>(a, st);
+  }
 }
 
 bool raytap_shape_ok(int C, int Cout) {
@@ -789,14 +813,10 @@ extern "C" int shrimp_conv_ln_raytap(const shrimp_raytap_args* a, void* stream) 
                  "conv_ln_raytap: alpha / bias / ln params / weights must be 16-byte aligned");
   SHRIMP_REQUIRE(a->r_sn >= RAY_SLOT_COUNT && a->re_sn >= 12 && a->g_sn >= 1,
                  "conv_ln_raytap: ray_idx rows need 32 slots, reach rows 12 bytes");
-  const int waves = (a->N + 16 * RT_MB - 1) / (16 * RT_MB);
-  const size_t lds = (size_t)rt_rows_bytes(a->N, a->C, a->Cout, waves) +
-                     (size_t)RAY_STEPS * a->C * 2 + (size_t)waves * 64 * 8 * 4;
-  SHRIMP_REQUIRE(lds <= (size_t)max_lds_per_block(), "conv_ln_raytap: needs %zu bytes of LDS", lds);
   hipStream_t s = as_stream(stream);
   switch (a->C) {
-    case 64: return launch_raytap_cin<64>(*a, lds, s);
-    case 96: return launch_raytap_cin<96>(*a, lds, s);
-    default: return launch_raytap_cin<128>(*a, lds, s);
+    case 64: return launch_raytap_cin<64>(*a, s);
+    case 96: return launch_raytap_cin<96>(*a, s);
+    default: return launch_raytap_cin<128>(*a, s);
   }
 }

@@ -97,7 +97,8 @@ def pack_attn_qkv(qkv_w, qkv_b, ln_w, ln_b):
 def pack_attn_mlp(out_w, out_b, g_attn, ln_w, ln_b, fc1_w, fc1_b, fc2_w, fc2_b, g_mlp):
     """AttnBlock out_proj / LN2 / fc1 / fc2 / LayerScale parameters -> the
     fused MLP kernel's packed weights (per-channel factors folded in), or
-    None when the shape has no fused kernel (C != 128 or hidden != 2C)."""
+    None when the shape has no fused kernel (C not 96, 128 or 192, or hidden
+    != 2C)."""
 
     require_device(out_w, "pack_attn_mlp")
     c = int(out_w.shape[0])

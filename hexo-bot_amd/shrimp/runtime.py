@@ -276,15 +276,15 @@ class HipForward:
                     ln1w=f32(blk.ln1.weight), ln1b=f32(blk.ln1.bias), eps1=blk.ln1.eps,
                     qkv_w=pack_linear_weight(qkv_w.detach().to(device)), qkv_b=f32(qkv_b),
                     # LN1 + q/k/v as one kernel with LN1 folded into the
-                    # weights where it applies (C = 128); else None
+                    # weights where it applies (C = 96, 128, 192); else None
                     qkv=pack_attn_qkv(qkv_w.to(device), qkv_b.to(device), blk.ln1.weight,
                                       blk.ln1.bias),
                     out_w=lin_w(at.out_proj), out_b=f32(at.out_proj.bias),
                     ln2w=f32(blk.ln2.weight), ln2b=f32(blk.ln2.bias), eps2=blk.ln2.eps,
                     fc1_w=lin_w(blk.fc1), fc1_b=f32(blk.fc1.bias),
                     fc2_w=lin_w(blk.fc2), fc2_b=f32(blk.fc2.bias),
-                    # out_proj + MLP as one fused kernel where its weights fit
-                    # one workgroup's LDS (C = 128, hidden = 2C); else None
+                    # out_proj + MLP as one fused kernel: weights in one workgroup's
+                    # LDS (C = 128) or streamed through it (96, 192); else None
                     mlp=pack_attn_mlp(at.out_proj.weight, at.out_proj.bias, blk.ls_attn.gamma,
                                       blk.ln2.weight, blk.ln2.bias, blk.fc1.weight, blk.fc1.bias,
                                       blk.fc2.weight, blk.fc2.bias, blk.ls_mlp.gamma),

@@ -247,9 +247,10 @@ int shrimp_linear(const shrimp_linear_args* a, void* stream);
 /* ------------------------------------------------------------------------
  * Fused LayerNorm + q/k/v projection (RelPosAttention.forward q_proj /
  * k_proj / v_proj on AttnBlock's ln1, model.py:448-492, 508-514; replaces
- * shrimp_linear's QKV mode for C = 128):
+ * shrimp_linear's QKV mode for C = 96, 128 and 192):
  *   n = LN1(x[r]) ;  [q | k | v] = n @ Wqkv^T + bqkv   -> qkv (3, B, H, S, dpad)
- * with rows r = (b, s). The padding lanes d..dpad of qkv are not written.
+ * with rows r = (b, s). The padding lanes d..dpad of qkv are written
+ * (zeros) at C = 96 and 192 only.
  * shrimp_pack_attn_qkv folds LN1's affine into the weights (W diag(ln_w),
  * b + W ln_b) and writes MFMA fragments, the folded bias and the column sums
  * of the bf16 weights (used by shrimp_attn_fused) to `packed`

@@ -262,6 +262,38 @@ def test_conv_ln_raytap_row_counts(n_pad, kinds):
     _k1_check(coords, mask, 96, 96, 8, seed=n_pad + 1, relus=(True,))
 
 
+@pytest.mark.parametrize("n_pad,b", [(1, 3), (33, 5), (128, 300), (129, 256), (129, 257), (256, 257),
+                                     (257, 2), (384, 2), (385, 2)])
+@pytest.mark.parametrize("c,cout", [(64, 64), (96, 96), (128, 128)])
+def test_conv_ln_raytap_row_splits(c, cout, n_pad, b):
+    """32- and 64-row waves on both sides of the rule (row counts 128, 256, 384,
+    the compute unit count): the first and last positions of the batch against
+    the oracle, a position's bits the same alone as in the batch."""
+
+    from hexfield_eq import build_tap_reach, hex_conv_ln_raytap
+
+    gen = torch.Generator().manual_seed(n_pad + b + c)
+    x, w, bias, lnw, lnb, alpha, raylen, _ = _k1_inputs(np.zeros((b, n_pad, 2), dtype=np.int64),
+                                                        np.ones((b, n_pad), dtype=bool), c, cout, n_pad)
+    idx = torch.randint(0, n_pad + 1, (b, n_pad, 32), generator=gen, dtype=torch.int32)
+    gidx = torch.randint(0, n_pad + 1, (b, n_pad, 7), generator=gen)
+    m = torch.rand(b, n_pad, generator=gen) < 0.9
+    reach = build_tap_reach(raylen.to(DEV))
+    par = [t.to(DEV) for t in (w, bias, lnw, lnb)]
+
+    def run(sel):
+        return hex_conv_ln_raytap(x[sel].to(DEV), gidx[sel].to(DEV), m[sel].to(DEV), *par,
+                                  idx[sel].to(DEV), reach[sel], alpha.to(DEV), 1e-5, True, 8)
+
+    got = run(slice(0, b))
+    for p in (0, b - 1):
+        sel = slice(p, p + 1)
+        want = ohf.conv_ln_raytap(x[sel], gidx[sel], m[sel], w, bias, lnw, lnb, idx[sel],
+                                  reach[sel].cpu(), alpha, 1e-5, True, 8)
+        torch.testing.assert_close(got[sel].double().cpu(), want, atol=5e-3, rtol=0)
+        assert torch.equal(run(sel), got[sel])
+
+
 def test_conv_ln_raytap_bench_shape_samples():
     """B = 1024, N = 256, C = Cout = 128 (the bench workload): three positions
     against the oracle."""

@@ -60,6 +60,11 @@ constexpr int KC = 64;              // keys per chunk
 constexpr int MAX_OFFSETS = 57 * 57;
 constexpr int TU = 16;              // table rows a wave loads together
 constexpr int MAX_LUT_M = 28;       // (2 M + 1)^2 entries fit the same region
+// Below this an offset's rounding (2^-24 of it) is 1.5e-5 of a weight. Scoring
+// again leaves a few 2^-24 of the old offset in the new one, so offsets of up to
+// 1e29 settle within six times.
+constexpr float FAR_OFFSET = 256.f;
+constexpr int MAX_RESCORES = 8;
 
 typedef __attribute__((address_space(3))) void lds_dst_t;
 typedef __attribute__((address_space(3))) const unsigned char lds_cu8;
@@ -149,11 +154,15 @@ constexpr int stream_nkb() {
 }
 
 // NKB blocks of 16 keys from key k0, K and V rows at LDS bytes kbuf, vbuf;
-// bit kb of `special` (wave-uniform): block kb selects its biases per lane.
+// bit kb of `special` (wave-uniform): block kb selects its biases per lane. False
+// (with `again`): the offsets moved and the blocks are to be scored once more.
+// Scores formed as score - m carry m's rounding, so an offset that was far larger
+// than the one that replaces it (a first chunk of keys masked by -1e9, say) leaves
+// them without their digits: -1e9 in a pair table gave errors of 0.5.
 template <int D, int QB, int PATH, int NKB>
-SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
+SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
                              int k0, int L, int special, int kbuf, int vbuf, int lr, int lg,
-                             float scale, const unsigned (&pd)[QB][NKB]) {
+                             float scale, const unsigned (&pd)[QB][NKB], bool again) {
   constexpr int KS = D / 32, KD = D / 16, RB = 2 * D;
   f32x4 v[QB][NKB];
   const int ksw = swz<D>(lr);
@@ -237,14 +246,16 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
     bad |= t > 0.f || !(w.l[qb][0] > 0.f);
   }
   if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+    bool far = false;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      const float g = max_groups_swap(mx[qb]);
+      const float g = max_groups_swap(mx[qb]), m0 = fabsf(w.m[qb]);
       const bool seen = w.l[qb][0] > 0.f;
       // no live key yet: the offset goes to this block's maximum, if it has one
       const float delta = seen ? fmaxf(g, 0.f) : (g > 0.1f * AST_NEG_BIG ? g : 0.f);
       const float alpha = seen ? __builtin_amdgcn_exp2f(-delta) : 0.f;
       w.m[qb] += delta;
+      far |= m0 > FAR_OFFSET && m0 > 2.f * fabsf(w.m[qb]);
       const float c = -w.m[qb] * s.inv_scale, lsum = w.l[qb][0] * alpha;
       w.cinit[qb] = f32x4{c, c, c, c};
       w.l[qb] = f32x4{lsum, lsum, lsum, lsum};
@@ -255,6 +266,7 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[qb][kb][j] -= delta;
     }
+    if (again && __builtin_amdgcn_ballot_w64(far) != 0) return false;
   }
   u32x2 pf[QB][NKB];
 #pragma unroll
@@ -292,6 +304,7 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
         w.o[qb][kd] =
             mfma16x16x32(u32x4{v0[kd].x, v0[kd].y, v1[kd].x, v1[kd].y}, pp[qb], w.o[qb][kd]);
   }
+  return true;
 }
 
 // LDS layout (bytes): [K, V chunk 0][K, V chunk 1][tables][kkey 4 SC or kqr 8 SC]
@@ -579,7 +592,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
           special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)lds_u8(lds_addr(flags) + c));
         }
 #pragma unroll 1
-        for (int kb = 0; kb < 4 && c * KC + kb * 16 < L; kb += NKB) {
+        for (int kb = 0, n = 0; kb < 4 && c * KC + kb * 16 < L;) {
           unsigned p[QB][NKB];
           if constexpr (PAIR) {
 #pragma unroll
@@ -587,9 +600,11 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
 #pragma unroll
               for (int i = 0; i < NKB; ++i) p[qb][i] = kb == 0 ? pd[qb][i] : pd[qb][(4 - NKB) + i];
           }
-          stream_chunk<D, QB, decltype(path)::value, NKB>(
+          const bool done = stream_chunk<D, QB, decltype(path)::value, NKB>(
               a, w, s, c * KC + kb * 16, L, special >> kb, kbuf + kb * 16 * RB, vbuf + kb * 16 * RB,
-              lr, lg, scale, p);
+              lr, lg, scale, p, n < MAX_RESCORES);
+          kb += done ? NKB : 0;
+          n = done ? 0 : n + 1;
           __builtin_amdgcn_sched_barrier(0);
         }
       }

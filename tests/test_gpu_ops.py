@@ -1314,6 +1314,33 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
 
 
+# Rows whose first keys (more than a chunk of 64) carry a mask of a large negative
+# bias: the offset that these set must not cost the later keys their digits. Both
+# query tilings of the streamed kernel (16 and 32 queries per wave), a ragged bound.
+@pytest.mark.parametrize("B", [3, 64])
+@pytest.mark.parametrize("low", [-65504.0, -1e9])
+@pytest.mark.parametrize("d", [16, 24, 32, 64])
+def test_attn_pair_low_first_keys(B, d, low):
+    g = torch.Generator().manual_seed(7)
+    H, S, rows = 4, 200, 238
+    q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
+    table2 = torch.randn(rows, H, generator=g) * 0.5
+    table2[rows - 1] = low
+    pair = torch.randint(0, rows - 1, (B, S, S), generator=g).to(torch.uint8)
+    pair[:, :, :100] = rows - 1
+    lens = torch.full((B,), S, dtype=torch.int32)
+    lens[1] = 150
+    dev = lambda t: t.to(DEV, torch.bfloat16)
+    got = torch.ops.shrimp.attn_pair(dev(q), dev(k), dev(v), pair.to(DEV), table2.to(DEV),
+                                     lens.to(DEV)).cpu().double()
+    want = ofwd.attn_pair(q, k, v, pair, table2.double(), lens)
+    # weights and result rounded to bf16: 2^-8 / sqrt(3) of a mantissa of 1 each,
+    # 1.66e-3 over random mantissas, 2.3e-3 together
+    err = ((got - want).norm() / want.norm()).item()
+    print(f"attn_pair B={B} d={d} low={low}: rel err {err:.3e}", flush=True)
+    assert err <= 2.5e-3
+
+
 # the weight-streamed conv (96 and 192 channels, their 32-channel stems): a last
 # tile of one row, a wave with no rows, and both row tilings (16 rows per wave
 # below 128 rows per compute unit, 32 from there); the K order and epilogue

@@ -1296,14 +1296,25 @@ int attn_rows_bf16(const shrimp_attn_args* a, hipStream_t st);
 // Keys streamed through LDS (attn_stream.hip): padded head dims 32 and 64.
 bool attn_stream_ok(const shrimp_attn_args* a, int npos);
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
-                       uint32_t o_bytes, hipStream_t st);
+                       uint32_t o_bytes, bool fine, hipStream_t st);
 
 template <bool PAIR>
 static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_bytes, int npos,
                          int tab_rows, hipStream_t st) {
   if (g_attn_variant == 3) return attn_rows_bf16(a, st);
-  if (attn_stream_ok(a, npos))
-    return launch_attn_stream(a, qk_scale, qkv_bytes, npos, attn_out_bytes(a), st);
+  if (attn_stream_ok(a, npos)) {
+    // Weights as two bf16 numbers where one would be less exact than the kernel that
+    // stood here (relative error against float64, of which the output's own rounding
+    // is 1.66e-3): past the whole-sequence kernels' sequences, where the chunked kernel
+    // keeps fp32 weights (1.66e-3; one bf16 2.12e-3), and short pair sequences, where
+    // a maximum per 16 keys instead of 64 leaves more weights exactly 1 (20, 68 and
+    // 128 rows 1.92e-3, 1.98e-3, 2.03e-3; one bf16 0.4, 1.2 and 0.2 % more, from 341
+    // rows the same). Two cost a tenth of the kernel: 111 positions, S = 584, H = 3,
+    // D = 64 94 -> 107 us.
+    const bool fine = (PAIR && a->S <= 256) ||
+                      attn_smem_bytes(a->dpad, 1, a->S, tab_rows, PAIR) > (size_t)max_lds_per_block();
+    return launch_attn_stream(a, qk_scale, qkv_bytes, npos, attn_out_bytes(a), fine, st);
+  }
 #define SHRIMP_ATTN_DP(DPV)                                                                \
   if (a->dpad == DPV) {                                                                    \
     const size_t s2 = attn_smem_bytes(DPV, 2, a->S, tab_rows, PAIR);                       \

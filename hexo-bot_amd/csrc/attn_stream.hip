@@ -159,7 +159,7 @@ constexpr int stream_nkb() {
 // Scores formed as score - m carry m's rounding, so an offset that was far larger
 // than the one that replaces it (a first chunk of keys masked by -1e9, say) leaves
 // them without their digits: -1e9 in a pair table gave errors of 0.5.
-template <int D, int QB, int PATH, int NKB>
+template <int D, int QB, int PATH, int NKB, bool FINE>
 SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
                              int k0, int L, int special, int kbuf, int vbuf, int lr, int lg,
                              float scale, const unsigned (&pd)[QB][NKB], bool again) {
@@ -268,7 +268,7 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
     }
     if (again && __builtin_amdgcn_ballot_w64(far) != 0) return false;
   }
-  u32x2 pf[QB][NKB];
+  u32x2 pf[QB][NKB], pl[QB][FINE ? NKB : 1];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
@@ -276,7 +276,11 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
       float p[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(v[qb][kb][j]);
-      pf[qb][kb] = u32x2{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+      const u32x2 hi{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+      pf[qb][kb] = hi;
+      if constexpr (FINE)
+        pl[qb][kb] = u32x2{pack_bf16x2(p[0] - bf16_lo(hi.x), p[1] - bf16_hi(hi.x)),
+                           pack_bf16x2(p[2] - bf16_lo(hi.y), p[3] - bf16_hi(hi.y))};
     }
   __builtin_amdgcn_sched_barrier(0);
   const unsigned one2 = 0x3F803F80u;
@@ -285,11 +289,15 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
   const int vlane = vbuf + vrow * RB + (lr & 1) * 8;
 #pragma unroll
   for (int kp = 0; kp < NKB; kp += 2) {
-    u32x4 pp[QB];
+    u32x4 pp[QB], pm[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       pp[qb] = u32x4{pf[qb][kp].x, pf[qb][kp].y, pf[qb][kp + 1].x, pf[qb][kp + 1].y};
       w.l[qb] = mfma16x16x32(u32x4{one2, one2, one2, one2}, pp[qb], w.l[qb]);
+      if constexpr (FINE) {
+        pm[qb] = u32x4{pl[qb][kp].x, pl[qb][kp].y, pl[qb][kp + 1].x, pl[qb][kp + 1].y};
+        w.l[qb] = mfma16x16x32(u32x4{one2, one2, one2, one2}, pm[qb], w.l[qb]);
+      }
     }
     int at[KD];
     u32x2 v0[KD], v1[KD];
@@ -300,9 +308,11 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
 #pragma unroll
     for (int kd = 0; kd < KD; ++kd)
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb)
-        w.o[qb][kd] =
-            mfma16x16x32(u32x4{v0[kd].x, v0[kd].y, v1[kd].x, v1[kd].y}, pp[qb], w.o[qb][kd]);
+      for (int qb = 0; qb < QB; ++qb) {
+        const u32x4 vf{v0[kd].x, v0[kd].y, v1[kd].x, v1[kd].y};
+        w.o[qb][kd] = mfma16x16x32(vf, pp[qb], w.o[qb][kd]);
+        if constexpr (FINE) w.o[qb][kd] = mfma16x16x32(vf, pm[qb], w.o[qb][kd]);
+      }
   }
   return true;
 }
@@ -315,7 +325,7 @@ __host__ __device__ inline int stream_tab_bytes(bool pair, int npos) {
   return pair ? (npos * 4 + 15) / 16 * 16 : (MAX_OFFSETS * 4 + 15) / 16 * 16;
 }
 
-template <int D, int QB, bool PAIR>
+template <int D, int QB, bool PAIR, bool FINE>
 __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const shrimp_attn_args a, float scale,
                                                              uint32_t qkv_bytes, int npos,
                                                              uint32_t o_bytes, int tiles) {
@@ -600,7 +610,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
 #pragma unroll
               for (int i = 0; i < NKB; ++i) p[qb][i] = kb == 0 ? pd[qb][i] : pd[qb][(4 - NKB) + i];
           }
-          const bool done = stream_chunk<D, QB, decltype(path)::value, NKB>(
+          const bool done = stream_chunk<D, QB, decltype(path)::value, NKB, FINE>(
               a, w, s, c * KC + kb * 16, L, special >> kb, kbuf + kb * 16 * RB, vbuf + kb * 16 * RB,
               lr, lg, scale, p, n < MAX_RESCORES);
           kb += done ? NKB : 0;
@@ -641,31 +651,37 @@ bool attn_stream_ok(const shrimp_attn_args* a, int npos) {
   return stream_smem(a->dpad, a->pair != nullptr, a->S, npos) <= (size_t)max_lds_per_block();
 }
 
-template <int D, int QB, bool PAIR>
+template <int D, int QB, bool PAIR, bool FINE>
 static int launch_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
                          uint32_t o_bytes, hipStream_t st) {
   const int tiles = (a->S + 64 * QB - 1) / (64 * QB);
-  hipLaunchKernelGGL((attn_stream_kernel<D, QB, PAIR>), dim3(a->B * a->H * tiles), dim3(256),
+  hipLaunchKernelGGL((attn_stream_kernel<D, QB, PAIR, FINE>), dim3(a->B * a->H * tiles), dim3(256),
                      stream_smem(D, PAIR, a->S, npos), st, *a, scale, qkv_bytes, npos, o_bytes, tiles);
   return check_launch("attn");
 }
 
 // 32 queries per wave (each K and V fragment read feeds two products) once
-// such tiles give every compute unit two workgroups, else 16.
+// such tiles give every compute unit two workgroups, else 16. fine: weights
+// as two bf16 numbers, their product with V as two (dispatch_attn says where).
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
-                       uint32_t o_bytes, hipStream_t st) {
+                       uint32_t o_bytes, bool fine, hipStream_t st) {
   const bool wide = (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
   const bool pair = a->pair != nullptr;
-#define AST_LAUNCH(DV)                                                                            \
-  if (pair)                                                                                       \
-    return wide ? launch_stream<DV, 2, true>(a, scale, qkv_bytes, npos, o_bytes, st)              \
-                : launch_stream<DV, 1, true>(a, scale, qkv_bytes, npos, o_bytes, st);             \
-  return wide ? launch_stream<DV, 2, false>(a, scale, qkv_bytes, npos, o_bytes, st)               \
-              : launch_stream<DV, 1, false>(a, scale, qkv_bytes, npos, o_bytes, st)
+#define AST_LAUNCH(...)                                                                       \
+  do {                                                                                        \
+    if (fine) return launch_stream<__VA_ARGS__, true>(a, scale, qkv_bytes, npos, o_bytes, st); \
+    return launch_stream<__VA_ARGS__, false>(a, scale, qkv_bytes, npos, o_bytes, st);         \
+  } while (0)
   if (a->dpad == 64) {
-    AST_LAUNCH(64);
+    if (pair && wide) AST_LAUNCH(64, 2, true);
+    if (pair) AST_LAUNCH(64, 1, true);
+    if (wide) AST_LAUNCH(64, 2, false);
+    AST_LAUNCH(64, 1, false);
   }
-  AST_LAUNCH(32);
+  if (pair && wide) AST_LAUNCH(32, 2, true);
+  if (pair) AST_LAUNCH(32, 1, true);
+  if (wide) AST_LAUNCH(32, 2, false);
+  AST_LAUNCH(32, 1, false);
 #undef AST_LAUNCH
 }
 

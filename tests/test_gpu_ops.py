@@ -1314,15 +1314,55 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
 
 
+# Weights held as two bf16 numbers: sequences past the whole-sequence kernels
+# (their other kernel holds fp32 weights) and short pair sequences. The result's
+# rounding to bf16 alone is 2^-8 / sqrt(3) of a mantissa of 1, 1.66e-3 over random
+# mantissas; weights of one bf16 give 2.1e-3.
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("B,H,S,d", [(2, 3, 660, 64), (64, 3, 641, 64), (2, 2, 1300, 32), (40, 2, 1300, 32)])
+def test_attn_long_sequence_error(B, H, S, d, pair):
+    from shrimp import ops
+    from shrimp.geometry import CELL_LUT_M, cell_bias_lut
+
+    g = torch.Generator().manual_seed(S + B)
+    q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
+    table = torch.randn(237, H, generator=g)
+    lens = torch.randint(S // 2, S + 1, (B,), generator=g).to(torch.int32)
+    n = min(B, 3)  # positions compared
+    qd, kd, vd = (t.to(DEV, torch.bfloat16) for t in (q, k, v))
+    ld = lens.to(DEV)
+    if pair:
+        rows = torch.randint(0, 237, (B, S, S), generator=g, dtype=torch.uint8)
+        got = torch.ops.shrimp.attn_pair(qd, kd, vd, rows.to(DEV), table.to(DEV), ld)
+        want = ofwd.attn_pair(q[:n], k[:n], v[:n], rows[:n], table.double(), lens[:n])
+    else:
+        at = torch.stack([torch.randperm(1444, generator=g)[:S] for _ in range(B)])
+        coords = torch.stack([at // 38, at % 38], -1).to(torch.int32)
+        btab, xtab = ops.attn_bias_table(table.to(DEV), torch.from_numpy(cell_bias_lut()).to(DEV))
+        got = torch.empty_like(qd)
+        cd, md = coords.to(DEV), torch.ones(B, S, dtype=torch.uint8, device=DEV)
+        ops.launch_attn(q=qd, k=kd, v=vd, qkv_sb=H * S * d, qkv_sh=S * d, seq_lens=ld, o=got,
+                        o_sb=H * S * d, o_sh=S * d, o_sr=d, B=B, S=S, H=H, d=d, dpad=d, coords=cd,
+                        mask8=md, btab=btab, xtab=xtab, lut_m=CELL_LUT_M, n_tokens=0)
+        want = _coords_attention_ref(q[:n], k[:n], v[:n], coords[:n],
+                                     torch.ones(n, S, dtype=torch.bool), lens[:n], table, 0)
+    live = (torch.arange(S) < lens[:n, None])[:, None, :, None].expand_as(want)
+    g64, w64 = got[:n].cpu().double()[live], want[live]
+    err = ((g64 - w64).norm() / w64.norm()).item()
+    print(f"attention B={B} S={S} d={d} pair={pair}: rel err {err:.3e}", flush=True)
+    assert err <= 1.75e-3
+
+
 # Rows whose first keys (more than a chunk of 64) carry a mask of a large negative
 # bias: the offset that these set must not cost the later keys their digits. Both
-# query tilings of the streamed kernel (16 and 32 queries per wave), a ragged bound.
-@pytest.mark.parametrize("B", [3, 64])
+# query tilings of the streamed kernel (16 and 32 queries per wave) with weights of
+# two bf16 numbers (200 rows) and of one (300), a ragged bound.
+@pytest.mark.parametrize("B,S", [(3, 200), (64, 200), (3, 300), (64, 300)])
 @pytest.mark.parametrize("low", [-65504.0, -1e9])
 @pytest.mark.parametrize("d", [16, 24, 32, 64])
-def test_attn_pair_low_first_keys(B, d, low):
+def test_attn_pair_low_first_keys(B, S, d, low):
     g = torch.Generator().manual_seed(7)
-    H, S, rows = 4, 200, 238
+    H, rows = 4, 238
     q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
     table2 = torch.randn(rows, H, generator=g) * 0.5
     table2[rows - 1] = low
@@ -1337,7 +1377,7 @@ def test_attn_pair_low_first_keys(B, d, low):
     # weights and result rounded to bf16: 2^-8 / sqrt(3) of a mantissa of 1 each,
     # 1.66e-3 over random mantissas, 2.3e-3 together
     err = ((got - want).norm() / want.norm()).item()
-    print(f"attn_pair B={B} d={d} low={low}: rel err {err:.3e}", flush=True)
+    print(f"attn_pair B={B} S={S} d={d} low={low}: rel err {err:.3e}", flush=True)
     assert err <= 2.5e-3
 
 

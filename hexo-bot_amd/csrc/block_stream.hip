@@ -388,10 +388,10 @@ __global__ __launch_bounds__(BW * 64, 2) void mlp_stream_kernel(const shrimp_mlp
       u32x4 gf[MB];
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
-        gf[mb] = u32x4{pack_bf16x2(gelu_ex2(ah[mb][0][0]), gelu_ex2(ah[mb][0][1])),
-                       pack_bf16x2(gelu_ex2(ah[mb][0][2]), gelu_ex2(ah[mb][0][3])),
-                       pack_bf16x2(gelu_ex2(ah[mb][1][0]), gelu_ex2(ah[mb][1][1])),
-                       pack_bf16x2(gelu_ex2(ah[mb][1][2]), gelu_ex2(ah[mb][1][3]))};
+        gf[mb] = u32x4{pack_bf16x2(gelu_fine(ah[mb][0][0]), gelu_fine(ah[mb][0][1])),
+                       pack_bf16x2(gelu_fine(ah[mb][0][2]), gelu_fine(ah[mb][0][3])),
+                       pack_bf16x2(gelu_fine(ah[mb][1][0]), gelu_fine(ah[mb][1][1])),
+                       pack_bf16x2(gelu_fine(ah[mb][1][2]), gelu_fine(ah[mb][1][3]))};
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
         const u32x4 w = lds_frag(w2 + nb * 1024);

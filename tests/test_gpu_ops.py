@@ -1489,6 +1489,30 @@ def test_block_rows_weight_streamed(c, H, B, S):
     assert torch.equal(lo_d.cpu().double()[keep[:, :nt]], bf(lo)[keep[:, :nt]])
 
 
+# The GELU of the 96- and 192-channel MLP kernel alone: fc1 is its bias, fc2 picks
+# one hidden unit per channel, so an output is bf16(GELU(b1)): half a bf16 step
+# (at most 2^-8 of the value) and the fp32 error of the erf form (4.5e-7) from float64.
+@pytest.mark.parametrize("c", [96, 192])
+def test_block_mlp_gelu(c):
+    from shrimp import ops
+
+    S, z = 4, lambda *s: torch.zeros(*s, device=DEV)
+    x = torch.cat([torch.linspace(-12, 12, 4 * c - 3), torch.tensor([-1e3, -1e4, 1e4])])
+    for part in x.split(2 * c):
+        b1, seq = part.to(DEV), z(S, 2, c).to(torch.bfloat16)
+        for half in range(2):
+            w2 = z(c, 2 * c)
+            w2[:, half * c:(half + 1) * c] = torch.eye(c, device=DEV)
+            packed = ops.pack_attn_mlp(z(c, c), z(c), z(c) + 1, z(c) + 1, z(c), z(2 * c, c), b1, w2,
+                                       z(c), z(c) + 1)
+            ops.launch_attn_mlp(x=z(S, c).to(torch.bfloat16), x_sr=c, seq=seq[:, half], s_sr=2 * c,
+                                mask=torch.ones(S, dtype=torch.uint8, device=DEV), packed=packed,
+                                eps=1e-5, rows=S, C=c, hidden=2 * c)
+        want = 0.5 * part.double() * torch.erfc(-part.double() / math.sqrt(2))
+        err = (seq.reshape(S, 2 * c).cpu().double() - want).abs() - 2.0 ** -8 * want.abs()
+        assert err.max() <= 4.5e-7, part[err.max(0).values.argmax()]
+
+
 # every operand conversion of the operator calls in one launch: vector and
 # element loads (padded channels, a source off 16 bytes), tails of the index and
 # of a workgroup, both weight layouts, six jobs at once, no rows; special values

@@ -62,16 +62,6 @@ SHRIMP_DEV void wait_vm() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
-// Row statistics of 16 rows whose channels lie as x[..] in this lane and its
-// three lane-group partners.
-template <int C>
-SHRIMP_DEV void row_stats(float s, float q, float eps, float& rstd, float& nmr) {
-  const float mean = sum_groups_swap(s) * (1.0f / C);
-  const float ex2 = sum_groups_swap(q) * (1.0f / C);
-  rstd = rsqrtf(fmaxf(fmaf(-mean, mean, ex2), 0.f) + eps);
-  nmr = -mean * rstd;
-}
-
 // ---- packed weights: byte offsets -------------------------------------------------
 constexpr uint32_t qkv_bias_off(int C) { return (uint32_t)(3 * C * C * 2); }
 constexpr uint32_t qkv_pack_bytes(int C) { return qkv_bias_off(C) + 3 * C * 4; }
@@ -340,26 +330,27 @@ __global__ __launch_bounds__(BW * 64, 2) void mlp_stream_kernel(const shrimp_mlp
   // as the fc2 accumulators' start
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    float sj[4], qj[4];
+    // two passes over the registers: E[x^2] - mean^2 cancels for rows whose mean is
+    // large against their spread
+    f32x4 sj = acc[mb][0];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      sj[j] = acc[mb][0][j];
-      qj[j] = acc[mb][0][j] * acc[mb][0][j];
+    for (int nb = 1; nb < NB; ++nb) sj = sj + acc[mb][nb];
+    const float mean = sum_groups_swap((sj[0] + sj[1]) + (sj[2] + sj[3])) * (1.0f / C);
+    float qj[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int nb = 1; nb < NB; ++nb) {
-        sj[j] += acc[mb][nb][j];
-        qj[j] = fmaf(acc[mb][nb][j], acc[mb][nb][j], qj[j]);
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float u = acc[mb][nb][j] - mean;
+        qj[j] = fmaf(u, u, qj[j]);
       }
-    }
-    float rstd, nmr;
-    row_stats<C>((sj[0] + sj[1]) + (sj[2] + sj[3]), (qj[0] + qj[1]) + (qj[2] + qj[3]), a.eps, rstd, nmr);
+    const float rstd =
+        rsqrtf(sum_groups_swap((qj[0] + qj[1]) + (qj[2] + qj[3])) * (1.0f / C) + a.eps);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const f32x4 v0 = acc[mb][2 * ks], v1 = acc[mb][2 * ks + 1];
-      hf[mb][ks] = u32x4{pack_bf16x2(fmaf(v0[0], rstd, nmr), fmaf(v0[1], rstd, nmr)),
-                         pack_bf16x2(fmaf(v0[2], rstd, nmr), fmaf(v0[3], rstd, nmr)),
-                         pack_bf16x2(fmaf(v1[0], rstd, nmr), fmaf(v1[1], rstd, nmr)),
-                         pack_bf16x2(fmaf(v1[2], rstd, nmr), fmaf(v1[3], rstd, nmr))};
+      const f32x4 v0 = (acc[mb][2 * ks] - mean) * rstd, v1 = (acc[mb][2 * ks + 1] - mean) * rstd;
+      hf[mb][ks] = u32x4{pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v0[2], v0[3]),
+                         pack_bf16x2(v1[0], v1[1]), pack_bf16x2(v1[2], v1[3])};
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = acc[mb][nb] + bias(3 * C + nb * 16);

@@ -1513,6 +1513,34 @@ def test_block_mlp_gelu(c):
         assert err.max() <= 4.5e-7, part[err.max(0).values.argmax()]
 
 
+# LayerNorm 2 of that kernel on rows whose mean is large against their spread (1024
+# against 0.5): bf16 weights, LayerNorm and hidden values leave under 1e-2 of the
+# MLP's part of the row (E[x^2] - mean^2 in fp32 has lost most digits of 0.25 there).
+@pytest.mark.parametrize("c", [96, 192])
+def test_block_mlp_large_mean(c):
+    from shrimp import ops
+
+    g = torch.Generator().manual_seed(c)
+    S, F, D = 64, torch.nn.functional, lambda t: t.double()
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g) * std
+    x, wo = r(S, c), r(c, c, std=0.5 / math.sqrt(c))
+    w1, b1, w2 = r(2 * c, c, std=0.1), r(2 * c, std=0.1), r(c, 2 * c)
+    z, one = torch.zeros(c), torch.ones(c)
+    dv = lambda t: t.to(DEV)
+    packed = ops.pack_attn_mlp(*(dv(t) for t in (wo, z, one, one, z, w1, b1, w2, z, one)))
+    seq = torch.full((S, c), 1024.0, dtype=torch.bfloat16, device=DEV)
+    lo = torch.zeros(1, S, c, dtype=torch.bfloat16, device=DEV)  # every row a token row
+    ops.launch_attn_mlp(x=dv(x).to(torch.bfloat16), x_sr=c, seq=seq, s_sr=c,
+                        mask=torch.ones(S, dtype=torch.uint8, device=DEV), packed=packed, eps=1e-5,
+                        rows=S, C=c, hidden=2 * c, tok_lo=lo, S=S, n_tokens=S)
+    s1 = 1024 + bf(x) @ bf(wo).T
+    want = F.gelu(F.layer_norm(s1, (c,), eps=1e-5) @ D(w1).T + D(b1)) @ D(w2).T
+    got = seq.cpu().double() + lo[0].cpu().double() - s1
+    err = ((got - want).norm() / want.norm()).item()
+    print(f"mlp large mean c={c}: rel err {err:.3e}", flush=True)
+    assert err <= 1e-2
+
+
 # every operand conversion of the operator calls in one launch: vector and
 # element loads (padded channels, a source off 16 bytes), tails of the index and
 # of a workgroup, both weight layouts, six jobs at once, no rows; special values

@@ -318,9 +318,12 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
 }
 
 // LDS layout (bytes): [K, V chunk 0][K, V chunk 1][tables][kkey 4 SC or kqr 8 SC]
-// [kcls SC][flags], SC = S rounded up to whole chunks; coords mode only past
-// the tables. 51.6 KB at D = 64 and S = 584: three workgroups per compute unit.
+// [kcls SC][flags][span per wave], SC = S rounded up to whole chunks; coords mode
+// only past the tables. All of it dynamic, so stream_smem is what a launch needs.
+// 51.7 KB at D = 64 and S = 584: three workgroups per compute unit.
 __host__ __device__ inline int stream_keys(int S) { return (S + KC - 1) / KC * KC; }
+__host__ __device__ inline int stream_flag_bytes(int SC) { return (SC / KC + 15) / 16 * 16; }
+constexpr int SPAN_BYTES = 4 * 4 * 4;
 __host__ __device__ inline int stream_tab_bytes(bool pair, int npos) {
   return pair ? (npos * 4 + 15) / 16 * 16 : (MAX_OFFSETS * 4 + 15) / 16 * 16;
 }
@@ -333,7 +336,6 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
   constexpr int CB = KC * RB;         // bytes of one chunk's K (or V) rows
   constexpr int PPR = D / 8;          // 16-byte pieces per row
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  __shared__ int span_red[4][4];
 
   // consecutive ids on one XCD (workgroups are dealt to the 8 XCDs round-robin),
   // so the query tiles of a (position, head) read K and V through one L2
@@ -391,6 +393,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
   int* kkey = reinterpret_cast<int*>(kqr);
   unsigned char* kcls = reinterpret_cast<unsigned char*>(kqr + SC);
   unsigned char* flags = kcls + SC;  // per chunk: bit kb, key block kb holds a token or dead key
+  int(*span_red)[4] = reinterpret_cast<int(*)[4]>(flags + stream_flag_bytes(SC));
 
   const int64_t base = (int64_t)b * a.qkv_sb + (int64_t)h * a.qkv_sh;
   const __amdgpu_buffer_rsrc_t qrs = make_rsrc(a.q, qkv_bytes);
@@ -634,7 +637,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
 size_t stream_smem(int D, bool pair, int S, int npos) {
   const size_t SC = (size_t)stream_keys(S);
   return (size_t)4 * KC * 2 * D + stream_tab_bytes(pair, npos) +
-         (pair ? 0 : SC * 9 + (SC / KC + 15) / 16 * 16);
+         (pair ? 0 : SC * 9 + stream_flag_bytes((int)SC) + SPAN_BYTES);
 }
 
 }  // namespace

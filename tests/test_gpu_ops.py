@@ -1314,6 +1314,35 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
 
 
+# The longest sequences that the streamed kernel's key tables fit beside its chunks
+# (14 848 at head dim 32) and the first ones past them, which the chunked kernel
+# takes: only 200 keys are live, so the rows are those of a short sequence.
+@pytest.mark.parametrize("S", [14848, 14849, 14912, 14913])
+def test_attn_longest_streamed(S):
+    from shrimp import ops
+    from shrimp.geometry import CELL_LUT_M, cell_bias_lut
+
+    g = torch.Generator().manual_seed(S)
+    L, d = 200, 32
+    q, k, v = (bf(torch.randn(1, 1, L, d, generator=g)) for _ in range(3))
+    table = torch.randn(237, 1, generator=g)
+    at = torch.randperm(400, generator=g)[:L]
+    coords = torch.stack([at // 20, at % 20], -1).to(torch.int32)[None]
+    btab, xtab = ops.attn_bias_table(table.to(DEV), torch.from_numpy(cell_bias_lut()).to(DEV))
+    grow = lambda t: torch.nn.functional.pad(t, (0, 0, 0, S - L))
+    qd, kd, vd = (grow(t).to(DEV, torch.bfloat16) for t in (q, k, v))
+    cd, md = grow(coords).to(DEV), torch.ones(1, S, dtype=torch.uint8, device=DEV)
+    ld = torch.tensor([L], dtype=torch.int32, device=DEV)
+    out = torch.full((1, 1, S, d), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.launch_attn(q=qd, k=kd, v=vd, qkv_sb=S * d, qkv_sh=S * d, seq_lens=ld, o=out, o_sb=S * d,
+                    o_sh=S * d, o_sr=d, B=1, S=S, H=1, d=d, dpad=d, coords=cd, mask8=md, btab=btab,
+                    xtab=xtab, lut_m=CELL_LUT_M, n_tokens=0)
+    want = _coords_attention_ref(q, k, v, coords, torch.ones(1, L, dtype=torch.bool),
+                                 torch.tensor([L]), table, 0)
+    close(out[:, :, :L], want, what=f"attention S={S}")
+    assert (out[:, :, L:] == 0).all()
+
+
 # Weights held as two bf16 numbers: sequences past the whole-sequence kernels
 # (their other kernel holds fp32 weights) and short pair sequences. The result's
 # rounding to bf16 alone is 2^-8 / sqrt(3) of a mantissa of 1, 1.66e-3 over random

@@ -1302,7 +1302,7 @@ template <bool PAIR>
 static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_bytes, int npos,
                          int tab_rows, hipStream_t st) {
   if (g_attn_variant == 3) return attn_rows_bf16(a, st);
-  if (attn_stream_ok(a, npos)) {
+  if (g_attn_variant == 0 && attn_stream_ok(a, npos)) {
     // Weights as two bf16 numbers where one would be less exact than the kernel that
     // stood here (relative error against float64, of which the output's own rounding
     // is 1.66e-3): past the whole-sequence kernels' sequences, where the chunked kernel

@@ -89,8 +89,8 @@ int fill_tokens_check(const float* tokens, int n_tokens, int C, const void* seq,
 // global-gather kernel, 2 = LDS-staged (no big tiles), 3 = as 0 without the
 // small-batch row split.
 extern std::atomic<int> g_conv_variant;
-// Attention: 0 = automatic (two heads per workgroup when they fit), 1 = one
-// head per workgroup, 2 = two heads on four waves, 3 = the chunked kernel
+// Attention: 0 = automatic (keys streamed through LDS at padded head dims 32 and
+// 64, two heads per workgroup when they fit at 16), 1 = one head per workgroup, 2 = two heads on four waves, 3 = the chunked kernel
 // (keys streamed through LDS; otherwise used only for sequences that do not
 // fit one workgroup's LDS).
 extern std::atomic<int> g_attn_variant;

@@ -59,13 +59,15 @@ int shrimp_abi_version(void);
  * gather rows from global memory, 2 = LDS-staged rows with small tiles,
  * 3 = as 0 without the small-batch row split; other values only query.
  * Returns the previous setting. Process-wide.
- * shrimp_attn_variant: 0 = automatic (two heads per attention workgroup when
- * their K/V fit the 64 KiB budget, on eight waves at padded head dim 16, else
+ * shrimp_attn_variant: 0 = automatic (padded head dims 32 and 64: keys streamed
+ * through LDS 64 at a time, where the q / k / v rows lie on 16-byte boundaries,
+ * lut_m <= 28 and the tables fit the LDS; else two heads per attention workgroup
+ * when their K/V fit the 64 KiB budget, on eight waves at padded head dim 16, else
  * four; one head per workgroup with up to the device's per-workgroup LDS for
  * longer sequences; beyond that the chunked kernel of shrimp_attn_f32 on bf16
  * operands), 1 = one head per workgroup, 2 = two heads on four waves, 3 = the
- * chunked kernel; other values only query. Returns the previous setting.
- * Process-wide.
+ * chunked kernel, none of these three the streamed one; other values only query.
+ * Returns the previous setting. Process-wide.
  * shrimp_max_lds_per_block: LDS bytes one workgroup may allocate on the
  * current device (the staged conv needs (N + 1) * cin_pad * 2). */
 int shrimp_conv_variant(int variant);

@@ -53,10 +53,11 @@ def conv_variant(request):
 
 @pytest.fixture(params=[0, 1, 2, 3], ids=["auto", "one_head", "four_waves", "chunked"])
 def attn_variant(request):
-    """Runs an attention test with the automatic kernel choice (two heads per
-    workgroup; eight waves at head dim 16), with one head per workgroup, with
-    two heads on four waves, and with the chunked kernel (keys streamed
-    through LDS, the path of sequences too long for one workgroup's LDS)."""
+    """Runs an attention test with the automatic kernel choice (head dim 16: two
+    heads per workgroup on eight waves; 32 and 64: keys streamed through LDS by
+    matrix tiles), with one head per workgroup, with two heads on four waves,
+    and with the chunked kernel (one query row per thread, the path of sequences
+    too long for the others' LDS)."""
 
     from shrimp import _lib
 
@@ -1341,6 +1342,58 @@ def test_attn_longest_streamed(S):
                                  torch.tensor([L]), table, 0)
     close(out[:, :, :L], want, what=f"attention S={S}")
     assert (out[:, :, L:] == 0).all()
+
+
+# Calls at head dims 32 and 64 that the streamed kernel does not take: a base or a
+# head stride off 16 bytes, a table wider than its region.
+@pytest.mark.parametrize("how", ["base", "stride", "table"])
+@pytest.mark.parametrize("d", [32, 64])
+def test_attn_streamed_fallback(d, how):
+    from shrimp import ops
+
+    g = torch.Generator().manual_seed(d)
+    B, H, S, M = 3, 4, 70, 30 if how == "table" else 16
+    q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
+    coords = torch.randint(-20, 20, (B, S, 2), generator=g, dtype=torch.int32)
+    lens = torch.tensor([70, 61, 23], dtype=torch.int32)
+    mask = torch.arange(S)[None] < lens[:, None]
+    table = torch.randn((2 * M + 1) ** 2, H, generator=g) * 0.5
+    btab = (torch.cat([table, torch.zeros(3, H)]) * (1.0 / math.log(2.0))).to(DEV)
+    off, sh = 4 * (how == "base"), S * d + 4 * (how == "stride")
+
+    def place(t):  # (B, H) rows of S d elements, sh apart, off from the allocation's start
+        out = torch.empty(off + B * H * sh, dtype=torch.bfloat16, device=DEV)
+        out[off:].view(B, H, sh)[..., :S * d] = t.reshape(B, H, S * d).to(DEV, torch.bfloat16)
+        return out[off:]
+
+    qd, kd, vd = place(q), place(k), place(v)
+    out = torch.full((B, H, S, d), 7.0, dtype=torch.bfloat16, device=DEV)
+    cd, md, ld = coords.to(DEV), mask.to(DEV, torch.uint8), lens.to(DEV)
+    ops.launch_attn(q=qd, k=kd, v=vd, qkv_sb=H * sh, qkv_sh=sh, seq_lens=ld, o=out, o_sb=H * S * d,
+                    o_sh=S * d, o_sr=d, B=B, S=S, H=H, d=d, dpad=d, coords=cd, mask8=md, btab=btab,
+                    lut_m=M, n_tokens=0)
+    want = ofwd.attn_offset_table(q, k, v, coords, mask, table.double(), M)
+    close(out, want, atol=1e-2, what=f"d={d} {how}")
+
+
+# The pair form on both query tilings (B H ceil(S / 128) of two per compute unit and
+# below) at sequence lengths around the pair loader's four keys, a 16-key block, a
+# chunk and a wave's queries, to 256 rows with weights of two bf16 numbers and
+# past them of one; ragged bounds, an odd head count. Eight positions compared.
+@pytest.mark.parametrize("B,H", [(3, 3), (172, 3)])
+@pytest.mark.parametrize("S", [1, 3, 17, 63, 65, 129, 321])
+@pytest.mark.parametrize("d", [24, 64])
+def test_attn_pair_streamed(d, S, B, H):
+    g = torch.Generator().manual_seed(S * 1000 + B + d)
+    q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
+    table2 = torch.randn(230, H, generator=g)
+    pair = torch.randint(0, 256, (B, S, S), generator=g).to(torch.uint8)  # past the table: its last row
+    lens = torch.randint(1, S + 1, (B,), generator=g).to(torch.int32)
+    lens[0], lens[1], lens[2] = S, 0, max(S // 16 * 16, 1)
+    dev = lambda t: t.to(DEV, torch.bfloat16)
+    got = torch.ops.shrimp.attn_pair(dev(q), dev(k), dev(v), pair.to(DEV), table2.to(DEV), lens.to(DEV))
+    want = ofwd.attn_pair(q[:8], k[:8], v[:8], pair[:8].clamp(max=229), table2.double(), lens[:8])
+    close(got[:8], want.nan_to_num(0.0), atol=1e-2, what=f"attn_pair B={B} S={S} d={d}")
 
 
 # Weights held as two bf16 numbers: sequences past the whole-sequence kernels

@@ -764,7 +764,7 @@ extern "C" int shrimp_op_prep(const int64_t* words, int n_jobs, void* stream) {
     } else {
       SHRIMP_REQUIRE((op == OP_CONV_W_BF16 || op == OP_RAYTAP_W_F16) && dt == SHRIMP_DT_F32,
                      "op_prep: unknown job %lld of dtype %d", (long long)op, (int)dt);
-      SHRIMP_REQUIRE(rows <= 64 && width > 0 && width <= dw && dw % 32 == 0 && extra > 0 &&
+      SHRIMP_REQUIRE(width > 0 && width <= dw && dw % 32 == 0 && extra > 0 &&
                          extra % 16 == 0 && mul_sat({rows, dw, extra, 2}) < (int64_t)0x7FFF0000,
                      "op_prep: weight (%lld, %lld -> %lld, %lld)", (long long)rows, (long long)width,
                      (long long)dw, (long long)extra);

@@ -1623,6 +1623,25 @@ def test_block_mlp_large_mean(c):
     assert err <= 1e-2
 
 
+# any tap count, as the packing and the conv take it
+@pytest.mark.parametrize("taps", [1, 64, 65, 127])
+def test_hex_conv_tap_counts(taps):
+    g = torch.Generator().manual_seed(taps)
+    B, N, c = 2, 33, 64
+    x = bf(torch.randn(B, N, c, generator=g))
+    idx = torch.randint(0, N + 1, (B, N, taps), generator=g)
+    mask = torch.rand(B, N, generator=g) < 0.9
+    w, b = torch.randn(taps, c, c, generator=g) / math.sqrt(taps * c), torch.randn(c, generator=g)
+    dev = lambda t: t.to(DEV)
+    got = torch.ops.shrimp.hex_conv(dev(x).float(), dev(idx), dev(mask), dev(w), dev(b))
+    close(got, ofwd.hex_conv(x, idx, mask, bf(w), b.double()), what=f"{taps} taps")
+    ln = torch.ops.shrimp.hex_conv_ln(dev(x).float(), dev(idx), dev(mask), dev(w), dev(b),
+                                      torch.ones(c, device=DEV), torch.zeros(c, device=DEV), 1e-5, False)
+    want = ofwd.hex_conv(x, idx, torch.ones_like(mask), bf(w), b.double())
+    want = torch.nn.functional.layer_norm(want, (c,)) * mask[..., None]
+    close(ln, want, what=f"{taps} taps + LN")
+
+
 # every operand conversion of the operator calls in one launch: vector and
 # element loads (padded channels, a source off 16 bytes), tails of the index and
 # of a workgroup, both weight layouts, six jobs at once, no rows; special values

@@ -27,7 +27,8 @@ enum : int { A_QKV = 1, A_QKV_W, A_QKV_B, A_LN1W, A_LN1B, A_EPS1, A_MLP, A_OUT_W
 // Call words.
 enum : int { I_IDX, I_MASK8, I_COORDS, I_SEQ_LENS, I_SEQ_MASK, I_XIN, I_WORKSPACE, I_QKV, I_POLICY,
              I_VALUE, I_ML, I_B, I_N, I_FLAGS, I_WORDS };
-enum : int { F_STAGED = 1, F_QKV = 2, F_MLP = 4, F_BLOCK = 8, F_PAIR = 16, F_TAIL = 32, F_LINEAR_BIAS = 64 };
+enum : int { F_STAGED = 1, F_QKV = 2, F_MLP = 4, F_BLOCK = 8, F_PAIR = 16, F_TAIL = 32, F_LINEAR_BIAS = 64,
+             F_END = 128 };
 
 float bits(int64_t w) {
   const uint32_t u = (uint32_t)w;
@@ -74,25 +75,35 @@ Regions regions(const int64_t* net, int64_t B, int64_t N, int flags, bool own_qk
   return r;
 }
 
-bool shape_ok(const int64_t* net, int64_t B, int64_t N) {
-  const int64_t c = net[W_C], h = net[W_H], dp = net[W_DPAD], nt = net[W_TOKEN_ROWS];
-  return B > 0 && N > 0 && N < shrimp::kMaxDim && c > 0 && c <= 4096 && h > 0 && h <= c && dp > 0 &&
-         dp <= 4096 && nt > 0 && nt <= 4096 &&
+// Everything that is narrowed to int below, and row counts, inside int.
+bool shape_ok(const int64_t* net, int64_t B, int64_t N, int64_t flags) {
+  const int64_t c = net[W_C], h = net[W_H], d = net[W_D], dp = net[W_DPAD], nt = net[W_TOKEN_ROWS];
+  return B > 0 && N > 0 && N < shrimp::kMaxDim && flags >= 0 && flags < F_END && c > 0 && c <= 4096 &&
+         h > 0 && c % h == 0 && c / h == d && dp >= d && dp <= 4096 && nt > 0 && nt <= 4096 &&
+         net[W_LUT_M] >= 0 && net[W_LUT_M] <= 64 && net[W_BINS] > 0 && net[W_BINS] <= 4096 &&
+         shrimp::mul_sat({B, N + nt}) <= INT32_MAX &&
          shrimp::mul_sat({B, N + nt, 4, c > h * dp ? c : h * dp, 2}) < ((int64_t)1 << 40);
 }
 
 }  // namespace
 
 extern "C" int64_t shrimp_forward_bytes(const int64_t* net, int B, int N, int flags, int own_qkv) {
-  if (net == nullptr || !shape_ok(net, B, N)) return 0;
+  if (net == nullptr || !shape_ok(net, B, N, flags)) return 0;
   return regions(net, B, N, flags, own_qkv != 0).total;
 }
 
 extern "C" int shrimp_forward(const int64_t* net, const int64_t* io, void* stream) {
   SHRIMP_REQUIRE(net && io, "forward: null words");
   if (io[I_B] == 0) return SHRIMP_OK;
-  SHRIMP_REQUIRE(shape_ok(net, io[I_B], io[I_N]) && net[W_LAYERS] > 0 && net[W_LAYERS] <= 1024,
-                 "forward: bad shape (B %lld, N %lld)", (long long)io[I_B], (long long)io[I_N]);
+  SHRIMP_REQUIRE(shape_ok(net, io[I_B], io[I_N], io[I_FLAGS]) && net[W_LAYERS] > 0 &&
+                     net[W_LAYERS] <= 1 << 20,
+                 "forward: bad shape (B %lld, N %lld, C %lld, H %lld, d %lld, flags %lld)",
+                 (long long)io[I_B], (long long)io[I_N], (long long)net[W_C], (long long)net[W_H],
+                 (long long)net[W_D], (long long)io[I_FLAGS]);
+  for (int64_t i = 0; i < net[W_LAYERS]; ++i)
+    SHRIMP_REQUIRE((net[W_HEAD_END + i * L_WORDS + L_KIND] | 1) == 1, "forward: layer %d of kind %lld",
+                   (int)i, (long long)net[W_HEAD_END + i * L_WORDS + L_KIND]);
+  SHRIMP_REQUIRE(net[W_TOKENS] != 0 && io[I_SEQ_MASK] != 0, "forward: null tokens or sequence mask");
   SHRIMP_REQUIRE(io[I_WORKSPACE] != 0 && (io[I_WORKSPACE] & 255) == 0,
                  "forward: workspace must be 256-byte aligned");
   const int B = (int)io[I_B], N = (int)io[I_N], flags = (int)io[I_FLAGS];

@@ -6,6 +6,8 @@
 // its checks fails at its launch), and calls
 //   - the argument checks the Python tests rely on, with their messages;
 //   - every entry point that takes an argument struct with a null struct;
+//   - the entry points that take word tables with valid tables, with single words
+//     out of range or inconsistent, and with random words;
 //   - every entry point with many random argument sets drawn from boundary
 //     values (sizes around the supported limits, negative and overflowing
 //     values, null pointers).
@@ -177,6 +179,118 @@ void known_rejections() {
   expect(shrimp_attn_fused_supported(128, 8, 321, 16) == 0, "attn_fused S limit");
 }
 
+// shrimp_forward's words (csrc/forward.cpp): a valid network of two layers and call.
+constexpr int kNetHead = 29, kLayerWords = 21, kIoWords = 14;
+enum : int { N_LAYERS = 0, N_C, N_H, N_D, N_DPAD, N_TOKENS, N_LUT_M = 26, N_TOKEN_ROWS, N_BINS };
+enum : int { IO_SEQ_MASK = 4, IO_WORKSPACE = 6, IO_QKV = 7, IO_ML = 10, IO_B, IO_N, IO_FLAGS };
+
+struct ForwardWords {
+  int64_t net[kNetHead + 2 * kLayerWords], io[kIoWords];
+  ForwardWords() {
+    const int64_t p = (int64_t)(uintptr_t)g_buf;
+    for (int64_t& w : net) w = p;
+    for (int64_t& w : io) w = p;
+    net[N_LAYERS] = 2; net[N_C] = 128; net[N_H] = 8; net[N_D] = net[N_DPAD] = 16;
+    net[N_LUT_M] = 17; net[N_TOKEN_ROWS] = 8; net[N_BINS] = 65;
+    net[kNetHead] = 0; net[kNetHead + kLayerWords] = 1;
+    io[IO_QKV] = 0; io[IO_B] = 3; io[IO_N] = 64; io[IO_FLAGS] = 2 | 4 | 64;
+  }
+  int64_t bytes() const { return shrimp_forward_bytes(net, (int)io[IO_B], (int)io[IO_N], (int)io[IO_FLAGS], 1); }
+};
+
+// Word tables: sizes that leave int when narrowed, inconsistent heads, unknown
+// flags, layers and jobs.
+void word_tables() {
+  {
+    ForwardWords f;
+    expect(f.bytes() > 0, "forward_bytes of a valid call");
+    expect(shrimp_forward_bytes(nullptr, 3, 64, 0, 1) == 0, "forward_bytes null");
+    const int rc = shrimp_forward(f.net, f.io, nullptr);
+    check_rc(rc, "forward");
+    expect(rc == SHRIMP_ELAUNCH, "forward of a valid call reaches its first launch");
+    f.io[IO_B] = 0;
+    expect(shrimp_forward(f.net, f.io, nullptr) == SHRIMP_OK, "forward of no positions");
+  }
+  ForwardWords none;
+  expect_einval(shrimp_forward(nullptr, none.io, nullptr), "null", "forward null net");
+  expect_einval(shrimp_forward(none.net, nullptr, nullptr), "null", "forward null io");
+  struct { bool net; int word; int64_t value; const char* needle; } bad[] = {
+      {false, IO_B, -1, "shape"}, {false, IO_B, ((int64_t)1 << 32) + 1, "shape"},
+      {false, IO_B, INT64_MAX, "shape"}, {false, IO_N, 0, "shape"}, {false, IO_N, -5, "shape"},
+      {false, IO_N, ((int64_t)1 << 32) + 64, "shape"}, {false, IO_B, 40000000, "shape"},
+      {false, IO_FLAGS, -1, "shape"}, {false, IO_FLAGS, 128, "shape"},
+      {false, IO_FLAGS, (int64_t)1 << 32, "shape"}, {false, IO_WORKSPACE, 0, "workspace"},
+      {false, IO_WORKSPACE, (int64_t)(uintptr_t)g_buf + 16, "workspace"}, {false, IO_SEQ_MASK, 0, "null"},
+      {true, N_LAYERS, 0, "shape"}, {true, N_LAYERS, (1 << 20) + 1, "shape"}, {true, N_C, 0, "shape"},
+      {true, N_C, 8192, "shape"}, {true, N_H, 0, "shape"}, {true, N_H, 16, "shape"},
+      {true, N_D, 8, "shape"}, {true, N_D, ((int64_t)1 << 32) + 16, "shape"}, {true, N_DPAD, 12, "shape"},
+      {true, N_DPAD, (int64_t)1 << 32, "shape"}, {true, N_TOKEN_ROWS, 0, "shape"},
+      {true, N_LUT_M, (int64_t)1 << 32, "shape"}, {true, N_BINS, 0, "shape"}, {true, N_TOKENS, 0, "null"},
+      {true, kNetHead, 2, "layer 0"}, {true, kNetHead + kLayerWords, -1, "layer 1"}};
+  for (const auto& b : bad) {
+    ForwardWords f;
+    (b.net ? f.net : f.io)[b.word] = b.value;
+    expect_einval(shrimp_forward(f.net, f.io, nullptr), b.needle, "forward");
+    if (b.net && b.word < kNetHead && b.word != N_LAYERS && b.word != N_TOKENS)
+      expect(f.bytes() == 0, "forward_bytes of a bad network");
+  }
+  // a small width with rows past int, below the byte limit
+  ForwardWords f;
+  f.net[N_C] = 16; f.net[N_H] = 1;
+  f.io[IO_B] = 32000000; f.io[IO_N] = 64;
+  expect_einval(shrimp_forward(f.net, f.io, nullptr), "shape", "forward rows");
+
+  const int64_t p = (int64_t)(uintptr_t)g_buf;
+  expect_einval(shrimp_op_prep(nullptr, 1, nullptr), "null", "op_prep null");
+  expect(shrimp_op_prep(nullptr, 0, nullptr) == SHRIMP_OK, "op_prep no jobs");
+  const int64_t job[8] = {p, p, 0, SHRIMP_DT_F32, 4, 24, 32, 0};
+  expect_einval(shrimp_op_prep(job, 7, nullptr), "jobs", "op_prep job count");
+  expect_einval(shrimp_op_prep(job, -1, nullptr), "jobs", "op_prep job count");
+  struct { int word; int64_t value; } badj[] = {
+      {0, 0}, {1, 0}, {1, p + 8}, {2, 4}, {2, -1}, {2, (int64_t)1 << 32}, {2, 2}, {3, SHRIMP_DT_I64}, {3, 99},
+      {4, -1}, {4, (int64_t)1 << 40}, {5, 0}, {5, 33}, {6, 28}, {6, INT64_MAX}};
+  for (const auto& b : badj) {
+    int64_t j[8];
+    std::memcpy(j, job, sizeof j);
+    j[b.word] = b.value;
+    expect_einval(shrimp_op_prep(j, 1, nullptr), "op_prep", "op_prep");
+  }
+  const int64_t taps[8] = {p, p, 2, SHRIMP_DT_F32, 65, 64, 64, 64};
+  const int rc = shrimp_op_prep(taps, 1, nullptr);
+  check_rc(rc, "op_prep");
+  expect(rc == SHRIMP_ELAUNCH, "op_prep of 65 taps reaches its launch");
+}
+
+void fuzz_words(uint64_t seed, int iters) {
+  Fuzz fz(seed);
+  for (int it = 0; it < iters; ++it) {
+    ForwardWords f;  // a few words off a valid call
+    const int widths[] = {16, 32, 64, 96, 128, 192, 256};
+    f.net[N_C] = widths[fz.u(7)];
+    f.net[N_H] = 1 + (int64_t)fz.u(8);
+    f.net[N_D] = f.net[N_C] / f.net[N_H];
+    f.net[N_DPAD] = (f.net[N_D] + 15) / 16 * 16;
+    f.io[IO_FLAGS] = (int64_t)fz.u(128);
+    f.io[IO_B] = 1 + (int64_t)fz.u(600);
+    f.io[IO_N] = 1 + (int64_t)fz.u(700);
+    if (fz.u(2)) f.io[IO_ML] = 0;
+    for (uint64_t k = fz.u(3); k > 0; --k) {
+      if (fz.u(2)) f.net[fz.u(kNetHead)] = fz.u(2) ? fz.i64() : (int64_t)fz.i32();
+      else f.io[fz.u(kIoWords)] = fz.u(2) ? fz.i64() : (int64_t)fz.i32();
+    }
+    if (f.net[N_LAYERS] > 2) f.net[N_LAYERS] = 2;
+    (void)shrimp_forward_bytes(f.net, fz.i32(), fz.i32(), fz.i32(), (int)fz.u(2));
+    check_rc(shrimp_forward(f.net, f.io, nullptr), "forward");
+    int64_t jobs[6 * 8];
+    for (int j = 0; j < 6; ++j) {
+      const int64_t w[8] = {(int64_t)(uintptr_t)fz.ptr(), (int64_t)(uintptr_t)fz.ptr(), (int64_t)fz.u(5),
+                            (int64_t)fz.u(7), fz.i64(), fz.i32(), fz.i32(), fz.i32()};
+      std::memcpy(jobs + 8 * j, w, sizeof w);
+    }
+    check_rc(shrimp_op_prep(jobs, (int)fz.u(8) - 1, nullptr), "op_prep");
+  }
+}
+
 void null_structs() {
   expect_einval(shrimp_hex_conv(nullptr, nullptr), nullptr, "hex_conv null");
   expect_einval(shrimp_hex_conv_f32(nullptr, nullptr), nullptr, "hex_conv_f32 null");
@@ -343,6 +457,8 @@ int main(int argc, char** argv) {
   expect(shrimp_abi_version() == SHRIMP_ABI_VERSION, "abi version");
   known_rejections();
   null_structs();
+  word_tables();
+  fuzz_words(seed + 2, iters);
   fuzz_structs(seed, iters);
   fuzz_scalars(seed + 1, iters);
   std::printf("abi_asan: %ld calls: %ld ok, %ld rejected, %ld reached a launch; %d failures\n", g_calls,

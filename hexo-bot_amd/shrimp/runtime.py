@@ -202,13 +202,19 @@ class HipForward:
         # "cuda" and "cuda:<current>" are one device: keyed apart, a caller that
         # names it one way and tensors that name it the other would re-pack the
         # weights at every switch
-        index = torch.cuda.current_device() if device.index is None else device.index
-        # the module tree walked directly: net.parameters() builds a name and a
-        # set entry per parameter, 0.2 ms for a 12-block network
+        device = torch.device(device)
+        index = device.index
+        if index is None and device.type == "cuda":
+            index = torch.cuda.current_device()
+        # the module tree walked directly (each module once): net.parameters()
+        # builds a name and a set entry per parameter, 0.2 ms for a 12-block network
         key = [device.type, index, self.precision]
-        todo = [self.net]
+        todo, seen = [self.net], set()
         while todo:
             m = todo.pop()
+            if id(m) in seen:
+                continue
+            seen.add(id(m))
             for p in m._parameters.values():
                 if p is not None:
                     key.append(p.data_ptr())

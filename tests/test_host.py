@@ -294,3 +294,8 @@ def test_parameter_key_walks_every_module():
             p.add_(0)
         assert rt._param_key(dev) != before
     assert rt._param_key(dev) != key and rt._param_key(torch.device("cuda", 1)) != rt._param_key(dev)
+    # a device by name or index; a module that is registered twice, or inside itself
+    assert rt._param_key("cuda:0") == rt._param_key(0) == rt._param_key(dev)
+    net.conv_blocks[0].register_module("owner", net)
+    assert rt._param_key(dev) == rt._param_key("cuda:0")
+    assert rt._param_key("cpu") != rt._param_key(dev)

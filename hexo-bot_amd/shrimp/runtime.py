@@ -322,9 +322,10 @@ class HipForward:
 
     @staticmethod
     def _net_words(P):
-        """The packed network as shrimp_forward takes it (csrc/forward.cpp)."""
+        """The packed network as shrimp_forward takes it (csrc/forward.cpp), made
+        again where P is a copy: its tensors are not those the words point at."""
 
-        if P.words is None:
+        if P.words is None or P.words[5] != P.tokens.data_ptr():
             p, f = _lib.ptr, _lib.float_word
             head = lambda h: [p(h.rw), p(h.rb), p(h.hw), p(h.hb)]
             w = [len(P.layout), P.C, P.H, P.d, P.dpad, p(P.tokens), p(P.stem.w), p(P.stem.b),

@@ -299,3 +299,33 @@ def test_parameter_key_walks_every_module():
     net.conv_blocks[0].register_module("owner", net)
     assert rt._param_key(dev) == rt._param_key("cuda:0")
     assert rt._param_key("cpu") != rt._param_key(dev)
+
+
+def test_forward_words_follow_their_weights():
+    """The native forward's words hold addresses: a copy of the packed weights
+    (deepcopy of a network that has run) gets words of its own tensors."""
+
+    import copy
+    from types import SimpleNamespace
+
+    from shrimp.runtime import HipForward
+
+    t = lambda: torch.zeros(4)
+    conv = dict(w1=t(), b1=t(), ln1w=t(), ln1b=t(), eps1=1e-5, w2=t(), b2=t(), ln2w=t(), ln2b=t(),
+                eps2=1e-5, gamma=t())
+    attn = dict(qkv=t(), qkv_w=t(), qkv_b=t(), ln1w=t(), ln1b=t(), eps1=1e-5, mlp=None, out_w=t(),
+                out_b=t(), g_attn=t(), ln2w=t(), ln2b=t(), eps2=1e-5, fc1_w=t(), fc1_b=t(), fc2_w=t(),
+                fc2_b=t(), g_mlp=t(), btab_xtab=(t(), t()))
+    head = lambda: SimpleNamespace(rw=t(), rb=t(), hw=t(), hb=t())
+    packed = SimpleNamespace(
+        layout="CA", C=32, H=4, d=8, dpad=16, tokens=t(), words=None, value=head(), ml=head(),
+        stem=SimpleNamespace(w=t(), b=t(), lnw=t(), lnb=t(), eps=1e-5),
+        lnf=SimpleNamespace(w=t(), b=t(), eps=1e-5),
+        policy=SimpleNamespace(w=t(), b=t(), hw=t(), hb=t()),
+        convs=[SimpleNamespace(**conv)], attn=[SimpleNamespace(**attn)])
+    words = HipForward._net_words(packed)
+    assert HipForward._net_words(packed) is words and words[5] == packed.tokens.data_ptr()
+    twin = copy.deepcopy(packed)
+    own = HipForward._net_words(twin)
+    assert own[5] == twin.tokens.data_ptr() and not set(own[29:]) & {packed.convs[0].w1.data_ptr()}
+    assert HipForward._net_words(twin) is own and HipForward._net_words(packed) is words

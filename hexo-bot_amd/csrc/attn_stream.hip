@@ -154,98 +154,101 @@ constexpr int stream_nkb() {
 }
 
 // NKB blocks of 16 keys from key k0, K and V rows at LDS bytes kbuf, vbuf;
-// bit kb of `special` (wave-uniform): block kb selects its biases per lane. False
-// (with `again`): the offsets moved and the blocks are to be scored once more.
-// Scores formed as score - m carry m's rounding, so an offset that was far larger
-// than the one that replaces it (a first chunk of keys masked by -1e9, say) leaves
-// them without their digits: -1e9 in a pair table gave errors of 0.5.
+// bit kb of `special` (wave-uniform): block kb selects its biases per lane.
 template <int D, int QB, int PATH, int NKB, bool FINE>
-SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
+SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
                              int k0, int L, int special, int kbuf, int vbuf, int lr, int lg,
-                             float scale, const unsigned (&pd)[QB][NKB], bool again) {
+                             float scale, const unsigned (&pd)[QB][NKB]) {
   constexpr int KS = D / 32, KD = D / 16, RB = 2 * D;
   f32x4 v[QB][NKB];
   const int ksw = swz<D>(lr);
+  // scores against the offsets
+  auto score = [&]() {
 #pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
+    for (int kb = 0; kb < NKB; ++kb) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const u32x4 kf = lds_16(kbuf + (kb * 16 + lr) * RB + (((ks * 4 + lg) ^ ksw) << 4));
+      for (int ks = 0; ks < KS; ++ks) {
+        const u32x4 kf = lds_16(kbuf + (kb * 16 + lr) * RB + (((ks * 4 + lg) ^ ksw) << 4));
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb)
-        v[qb][kb] = mfma16x16x32(kf, w.qf[qb][ks], ks == 0 ? w.cinit[qb] : v[qb][kb]);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
-    const int key0 = k0 + kb * 16 + lg * 4;
-    u32x4 kk{0, 0, 0, 0}, kr{0, 0, 0, 0};
-    if constexpr (PATH == PATH_LINEAR) {
-      kk = lds_16(s.keys + key0 * 4);
-    } else if constexpr (PATH == PATH_CLAMP) {
-      const u32x4 a0 = lds_16(s.keys + key0 * 8), a1 = lds_16(s.keys + key0 * 8 + 16);
-      kk = u32x4{a0[0], a0[2], a1[0], a1[2]};
-      kr = u32x4{a0[1], a0[3], a1[1], a1[3]};
-    }
-    const int kv[4] = {(int)kk[0], (int)kk[1], (int)kk[2], (int)kk[3]};
-    const int rv[4] = {(int)kr[0], (int)kr[1], (int)kr[2], (int)kr[3]};
-    float bias[QB][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        if constexpr (PATH == PATH_LINEAR) {
-          bias[qb][j] = lds_f32(kv[j] - w.qkey[qb]);
-        } else if constexpr (PATH == PATH_CLAMP) {
-          const int M = a.lut_m, W = 2 * M + 1;
-          bias[qb][j] = lds_f32(
-              s.tab + ((clampi(kv[j] - w.qq[qb], M) + M) * W + clampi(rv[j] - w.qr[qb], M) + M) * 4);
-        } else {
-          const int p = (int)((pd[qb][kb] >> (8 * j)) & 0xFF);
-          bias[qb][j] = lds_f32(s.tab + min(p, s.npos - 1) * 4);
-        }
+        for (int qb = 0; qb < QB; ++qb)
+          v[qb][kb] = mfma16x16x32(kf, w.qf[qb][ks], ks == 0 ? w.cinit[qb] : v[qb][kb]);
       }
-    if ((special >> kb) & 1) {
-      unsigned cls = 0;
-      if constexpr (PATH != PATH_PAIR) cls = lds_u32(s.kcls + key0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = (cls >> (8 * j)) & 0xFF;
-        const bool dead = PATH == PATH_PAIR ? key0 + j >= L : c == KEY_DEAD;
+    for (int kb = 0; kb < NKB; ++kb) {
+      const int key0 = k0 + kb * 16 + lg * 4;
+      u32x4 kk{0, 0, 0, 0}, kr{0, 0, 0, 0};
+      if constexpr (PATH == PATH_LINEAR) {
+        kk = lds_16(s.keys + key0 * 4);
+      } else if constexpr (PATH == PATH_CLAMP) {
+        const u32x4 a0 = lds_16(s.keys + key0 * 8), a1 = lds_16(s.keys + key0 * 8 + 16);
+        kk = u32x4{a0[0], a0[2], a1[0], a1[2]};
+        kr = u32x4{a0[1], a0[3], a1[1], a1[3]};
+      }
+      const int kv[4] = {(int)kk[0], (int)kk[1], (int)kk[2], (int)kk[3]};
+      const int rv[4] = {(int)kr[0], (int)kr[1], (int)kr[2], (int)kr[3]};
+      float bias[QB][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-          if constexpr (PATH != PATH_PAIR) {
-            const float ct = w.qtok[qb] ? s.tokb[1] : bias[qb][j];
-            const float tt = w.qtok[qb] ? s.tokb[2] : s.tokb[0];
-            bias[qb][j] = c == KEY_TOKEN ? tt : ct;
+          if constexpr (PATH == PATH_LINEAR) {
+            bias[qb][j] = lds_f32(kv[j] - w.qkey[qb]);
+          } else if constexpr (PATH == PATH_CLAMP) {
+            const int M = a.lut_m, W = 2 * M + 1;
+            bias[qb][j] = lds_f32(
+                s.tab + ((clampi(kv[j] - w.qq[qb], M) + M) * W + clampi(rv[j] - w.qr[qb], M) + M) * 4);
+          } else {
+            const int p = (int)((pd[qb][kb] >> (8 * j)) & 0xFF);
+            bias[qb][j] = lds_f32(s.tab + min(p, s.npos - 1) * 4);
           }
-          // dead keys' K rows are zero, so this is their score: exp2 of it is 0
-          // against any offset (offsets are real scores)
-          if (dead) bias[qb][j] = AST_NEG_BIG;
+        }
+      if ((special >> kb) & 1) {
+        unsigned cls = 0;
+        if constexpr (PATH != PATH_PAIR) cls = lds_u32(s.kcls + key0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c = (cls >> (8 * j)) & 0xFF;
+          const bool dead = PATH == PATH_PAIR ? key0 + j >= L : c == KEY_DEAD;
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) {
+            if constexpr (PATH != PATH_PAIR) {
+              const float ct = w.qtok[qb] ? s.tokb[1] : bias[qb][j];
+              const float tt = w.qtok[qb] ? s.tokb[2] : s.tokb[0];
+              bias[qb][j] = c == KEY_TOKEN ? tt : ct;
+            }
+            // dead keys' K rows are zero, so this is their score: exp2 of it is 0
+            // against any offset (offsets are real scores)
+            if (dead) bias[qb][j] = AST_NEG_BIG;
+          }
         }
       }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) v[qb][kb][j] = fmaf(v[qb][kb][j], scale, bias[qb][j]);
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) v[qb][kb][j] = fmaf(v[qb][kb][j], scale, bias[qb][j]);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  // does any query's offset have to move?
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // largest score of each query in this lane; whether any offset has to move
   float mx[QB];
-  bool bad = false;
+  auto over = [&]() -> bool {
+    bool bad = false;
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb) {
-    float t = v[qb][0][0];
+    for (int qb = 0; qb < QB; ++qb) {
+      float t = v[qb][0][0];
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) t = fmaxf(t, v[qb][kb][j]);
-    mx[qb] = t;
-    bad |= t > 0.f || !(w.l[qb][0] > 0.f);
-  }
-  if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+        for (int j = 0; j < 4; ++j) t = fmaxf(t, v[qb][kb][j]);
+      mx[qb] = t;
+      bad |= t > 0.f || !(w.l[qb][0] > 0.f);
+    }
+    return __builtin_amdgcn_ballot_w64(bad) != 0;
+  };
+  // moves them; whether one fell far
+  auto shift = [&]() -> bool {
     bool far = false;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -266,7 +269,21 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[qb][kb][j] -= delta;
     }
-    if (again && __builtin_amdgcn_ballot_w64(far) != 0) return false;
+    return __builtin_amdgcn_ballot_w64(far) != 0;
+  };
+  score();
+  if (over()) {
+    bool far = shift();
+    // Scores formed as score - m carry m's rounding, so an offset far larger than the
+    // one that replaces it (a first chunk of keys masked by -1e9, say) leaves them
+    // without their digits: -1e9 in a pair table gave errors of 0.5. They are formed
+    // again around the new one.
+#pragma unroll 1
+    for (int n = 0; __builtin_expect(far, 0) && n < MAX_RESCORES; ++n) {
+      score();
+      (void)over();
+      far = shift();
+    }
   }
   u32x2 pf[QB][NKB], pl[QB][FINE ? NKB : 1];
 #pragma unroll
@@ -314,7 +331,6 @@ SHRIMP_DEV bool stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
         if constexpr (FINE) w.o[qb][kd] = mfma16x16x32(vf, pm[qb], w.o[qb][kd]);
       }
   }
-  return true;
 }
 
 // LDS layout (bytes): [K, V chunk 0][K, V chunk 1][tables][kkey 4 SC or kqr 8 SC]
@@ -605,7 +621,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
           special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)lds_u8(lds_addr(flags) + c));
         }
 #pragma unroll 1
-        for (int kb = 0, n = 0; kb < 4 && c * KC + kb * 16 < L;) {
+        for (int kb = 0; kb < 4 && c * KC + kb * 16 < L; kb += NKB) {
           unsigned p[QB][NKB];
           if constexpr (PAIR) {
 #pragma unroll
@@ -613,11 +629,9 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
 #pragma unroll
               for (int i = 0; i < NKB; ++i) p[qb][i] = kb == 0 ? pd[qb][i] : pd[qb][(4 - NKB) + i];
           }
-          const bool done = stream_chunk<D, QB, decltype(path)::value, NKB, FINE>(
+          stream_chunk<D, QB, decltype(path)::value, NKB, FINE>(
               a, w, s, c * KC + kb * 16, L, special >> kb, kbuf + kb * 16 * RB, vbuf + kb * 16 * RB,
-              lr, lg, scale, p, n < MAX_RESCORES);
-          kb += done ? NKB : 0;
-          n = done ? 0 : n + 1;
+              lr, lg, scale, p);
           __builtin_amdgcn_sched_barrier(0);
         }
       }

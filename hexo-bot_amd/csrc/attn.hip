@@ -1298,11 +1298,26 @@ bool attn_stream_ok(const shrimp_attn_args* a, int npos);
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
                        uint32_t o_bytes, bool fine, hipStream_t st);
 
+// Where the streamed kernel is the faster one at head dims 32 and 64: the pair form
+// everywhere; the coords form, whose workgroups each build the key codes and the bias
+// table that the whole-sequence kernel builds once for two heads, unless there are
+// enough heads to fill the device and sequences short enough for several
+// whole-sequence workgroups per compute unit. Streamed against whole-sequence, us:
+// H = 4, D = 32 B = 200, S = 136 25.6 / 18.6; B = 384, S = 200 52.5 / 47.3, S = 264
+// 84.0 / 70.4, S = 328 100.6 / 118.3; H = 3, D = 64 B = 400, S = 136 50 / 41, S = 176
+// 54 / 65. To 128 rows and from 1024 heads the streamed one again (B = 800, H = 4,
+// D = 32, S = 72 0.88 times, S = 128 0.86). Below 384 heads it is within 9 % or faster.
+static bool attn_stream_faster(const shrimp_attn_args* a) {
+  const int64_t heads = (int64_t)a->B * a->H;
+  if (a->pair != nullptr || 2 * heads < 3 * cu_count()) return true;
+  return a->S <= 128 ? heads >= 4 * cu_count() : a->S > 10240 / a->dpad;
+}
+
 template <bool PAIR>
 static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_bytes, int npos,
                          int tab_rows, hipStream_t st) {
   if (g_attn_variant == 3) return attn_rows_bf16(a, st);
-  if (g_attn_variant == 0 && attn_stream_ok(a, npos)) {
+  if (g_attn_variant == 0 && attn_stream_ok(a, npos) && attn_stream_faster(a)) {
     // Weights as two bf16 numbers where one would be less exact than the kernel that
     // stood here (relative error against float64, of which the output's own rounding
     // is 1.66e-3): past the whole-sequence kernels' sequences, where the chunked kernel

@@ -677,25 +677,32 @@ static int launch_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_by
   return check_launch("attn");
 }
 
-// 32 queries per wave (each K and V fragment read feeds two products) once
-// such tiles give every compute unit two workgroups, else 16. fine: weights
-// as two bf16 numbers, their product with V as two (dispatch_attn says where).
+// 32 queries per wave (each K and V fragment read feeds two products) for a coords
+// call of more than 64 rows once such tiles give every compute unit two workgroups,
+// else 16. Measured, 16 against 32: coords at 768 positions, H = 4, D = 32 200 rows
+// 1.27 times the time, 328 rows 1.32, 64 rows (half of a 128-query tile empty) 0.88.
+// The pair form, whose scores wait for their pair rows, takes 32 only where one tile
+// of 128 stands for two of 64 (72 rows, 512 positions, H = 4, D = 32 26.7 us with 16,
+// 22.6 with 32; from 104 rows 0.71 to 1.02 times the time with 16). fine: weights as
+// two bf16 numbers, their product with V as two (dispatch_attn says where; a pair
+// call of at most 256 rows always).
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
                        uint32_t o_bytes, bool fine, hipStream_t st) {
-  const bool wide = (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
   const bool pair = a->pair != nullptr;
+  const bool wide = a->S > 64 && (!pair || a->S <= 96) &&
+                    (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
 #define AST_LAUNCH(...)                                                                       \
   do {                                                                                        \
     if (fine) return launch_stream<__VA_ARGS__, true>(a, scale, qkv_bytes, npos, o_bytes, st); \
     return launch_stream<__VA_ARGS__, false>(a, scale, qkv_bytes, npos, o_bytes, st);         \
   } while (0)
   if (a->dpad == 64) {
-    if (pair && wide) AST_LAUNCH(64, 2, true);
+    if (pair && wide) return launch_stream<64, 2, true, true>(a, scale, qkv_bytes, npos, o_bytes, st);
     if (pair) AST_LAUNCH(64, 1, true);
     if (wide) AST_LAUNCH(64, 2, false);
     AST_LAUNCH(64, 1, false);
   }
-  if (pair && wide) AST_LAUNCH(32, 2, true);
+  if (pair && wide) return launch_stream<32, 2, true, true>(a, scale, qkv_bytes, npos, o_bytes, st);
   if (pair) AST_LAUNCH(32, 1, true);
   if (wide) AST_LAUNCH(32, 2, false);
   AST_LAUNCH(32, 1, false);

@@ -1268,7 +1268,9 @@ def _coords_attention_ref(q, k, v, coords, mask, lens, table, nt):
 
 # head dims 32 and 64 stream the keys through LDS 64 at a time: sequence
 # lengths around a chunk and around the two query tilings (64 queries per
-# workgroup, or 128 once B H tiles reach two per compute unit: B = 96, H = 6),
+# workgroup, or 128 past 64 rows once B H tiles reach two per compute unit; at most
+# 320 rows at head dim 32 and 160 at 64 that is from 1024 heads, the whole-sequence
+# kernels taking 384 to 1024),
 # spans on either side of the unclamped table (window 20: linear, 60: clamped),
 # lengths of 0, inside the tokens and ragged, dead cells whose K and V rows hold
 # NaN, a head dim below its padding, an odd head count
@@ -1276,7 +1278,8 @@ def _coords_attention_ref(q, k, v, coords, mask, lens, table, nt):
 @pytest.mark.parametrize("B,H,S,d,dpad,nt,window", [
     (5, 3, 64, 64, 64, 8, 20), (5, 3, 65, 64, 64, 8, 60), (5, 4, 130, 24, 32, 8, 20),
     (5, 4, 63, 32, 32, 0, 60), (96, 6, 72, 32, 32, 8, 20), (96, 6, 129, 64, 64, 0, 60),
-    (5, 3, 584, 64, 64, 8, 40),
+    (5, 3, 584, 64, 64, 8, 40), (172, 6, 72, 32, 32, 8, 20), (172, 6, 127, 64, 64, 0, 60),
+    (60, 3, 330, 32, 32, 8, 40), (90, 3, 257, 64, 64, 0, 60),
 ])
 def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     from shrimp import ops
@@ -1376,12 +1379,12 @@ def test_attn_streamed_fallback(d, how):
     close(out, want, atol=1e-2, what=f"d={d} {how}")
 
 
-# The pair form on both query tilings (B H ceil(S / 128) of two per compute unit and
-# below) at sequence lengths around the pair loader's four keys, a 16-key block, a
+# The pair form on both query tilings (128 queries per workgroup from 65 to 96 rows
+# once those are two per compute unit: B = 172, H = 3) at sequence lengths around the pair loader's four keys, a 16-key block, a
 # chunk and a wave's queries, to 256 rows with weights of two bf16 numbers and
 # past them of one; ragged bounds, an odd head count. Eight positions compared.
 @pytest.mark.parametrize("B,H", [(3, 3), (172, 3)])
-@pytest.mark.parametrize("S", [1, 3, 17, 63, 65, 129, 321])
+@pytest.mark.parametrize("S", [1, 3, 17, 63, 65, 96, 97, 129, 321])
 @pytest.mark.parametrize("d", [24, 64])
 def test_attn_pair_streamed(d, S, B, H):
     g = torch.Generator().manual_seed(S * 1000 + B + d)
@@ -1436,9 +1439,8 @@ def test_attn_long_sequence_error(B, H, S, d, pair):
 
 
 # Rows whose first keys (more than a chunk of 64) carry a mask of a large negative
-# bias: the offset that these set must not cost the later keys their digits. Both
-# query tilings of the streamed kernel (16 and 32 queries per wave) with weights of
-# two bf16 numbers (200 rows) and of one (300), a ragged bound.
+# bias: the offset that these set must not cost the later keys their digits. Weights
+# of two bf16 numbers (200 rows) and of one (300), a ragged bound.
 @pytest.mark.parametrize("B,S", [(3, 200), (64, 200), (3, 300), (64, 300)])
 @pytest.mark.parametrize("low", [-65504.0, -1e9])
 @pytest.mark.parametrize("d", [16, 24, 32, 64])

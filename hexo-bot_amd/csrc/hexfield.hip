@@ -697,14 +697,18 @@ int launch_ray_attn(const shrimp_ray_attn_args& a, bool stage, hipStream_t st) {
 template <int CIN, int COUT>
 int launch_raytap(const shrimp_raytap_args& a, hipStream_t st) {
   // 64-row waves where those fill a compute unit already (two workgroups of three
-  // or four waves at 242-256 VGPRs; 32-row waves at 128 VGPRs, Cout = 64, fit four
-  // per SIMD and win there too) and past the 32-row waves' 384 rows. Measured, 64
-  // against 32 rows, C = Cout: 96 channels B = 200, N = 300 38.9 / 30.3 us; B = 512,
-  // N = 300 78.5 / 62.4; B = 256, N = 256 31.1 / 25.0, B = 260 39.6 / 44.4; B = 1024,
-  // N = 256 83.9 / 95.1, N = 128 47.4 / 46.9, N = 64 32.4 / 26.4. 128 channels
-  // B = 8, N = 256 35.7 / 29.0; B = 1024, N = 256 112.1 / 128.9. 64 channels
-  // B = 1024, N = 256 55.9 / 55.0.
-  const bool full = COUT > 64 && a.N > 128 && a.N <= 256 && a.B > cu_count();
+  // or four waves at 242-256 VGPRs; Cout = 64 at 159-174 VGPRs three, and its 32-row
+  // waves at 128 need a second round from three workgroups per unit to 192 rows, from
+  // four to 240) and past the 32-row waves' 384 rows. Measured, 64 against 32 rows,
+  // C = Cout: 96 channels B = 200, N = 300 38.9 / 30.3 us; B = 512, N = 300 78.5 / 62.4,
+  // N = 384 81.6 / 67.2; B = 256, N = 256 31.1 / 25.0, B = 260 39.6 / 44.4; B = 1024,
+  // N = 256 83.9 / 95.1, N = 128 47.4 / 46.9, N = 64 32.4 / 26.4. 128 channels B = 8,
+  // N = 256 35.7 / 29.0; B = 700, N = 384 159 / 135; B = 1024, N = 256 112.1 / 128.9.
+  // 64 channels B = 768, N = 192 39.8 / 38.0, B = 800 41.1 / 50.3, B = 1024 43.0 / 59.4;
+  // N = 224, B = 1024 51.6 / 50.0, B = 1500 69.9 / 82.1; N = 256 73.1 / 73.7.
+  const int64_t cus = cu_count();
+  const bool full = a.N > 128 && a.N <= 256 &&
+                    (COUT > 64 ? a.B > cus : a.N <= 240 && a.B > (a.N <= 192 ? 3 : 4) * cus);
   const int mb = full || a.N > RT_HALF_N ? 4 : 2;
   const int waves = (a.N + 16 * mb - 1) / (16 * mb);
   const size_t lds = (size_t)rt_rows_bytes(a.N, CIN, COUT, waves * 16 * mb) +

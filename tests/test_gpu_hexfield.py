@@ -263,11 +263,11 @@ def test_conv_ln_raytap_row_counts(n_pad, kinds):
 
 
 @pytest.mark.parametrize("n_pad,b", [(1, 3), (33, 5), (128, 300), (129, 256), (129, 257), (256, 257),
-                                     (257, 2), (384, 2), (385, 2)])
+                                     (257, 2), (384, 2), (385, 2), (160, 768), (160, 769), (240, 1025)])
 @pytest.mark.parametrize("c,cout", [(64, 64), (96, 96), (128, 128)])
 def test_conv_ln_raytap_row_splits(c, cout, n_pad, b):
     """32- and 64-row waves on both sides of the rule (row counts 128, 256, 384,
-    the compute unit count): the first and last positions of the batch against
+    one, three and four positions per compute unit): the first and last positions of the batch against
     the oracle, a position's bits the same alone as in the batch."""
 
     from hexfield_eq import build_tap_reach, hex_conv_ln_raytap

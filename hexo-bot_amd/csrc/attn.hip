@@ -1325,7 +1325,7 @@ static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv
     // a maximum per 16 keys instead of 64 leaves more weights exactly 1 (20, 68 and
     // 128 rows 1.92e-3, 1.98e-3, 2.03e-3; one bf16 0.4, 1.2 and 0.2 % more, from 341
     // rows the same). Two cost a tenth of the kernel: 111 positions, S = 584, H = 3,
-    // D = 64 94 -> 107 us.
+    // D = 64 94 -> 106 us.
     const bool fine = (PAIR && a->S <= 256) ||
                       attn_smem_bytes(a->dpad, 1, a->S, tab_rows, PAIR) > (size_t)max_lds_per_block();
     return launch_attn_stream(a, qk_scale, qkv_bytes, npos, attn_out_bytes(a), fine, st);

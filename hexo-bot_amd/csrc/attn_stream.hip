@@ -23,9 +23,10 @@
 // accumulators start at -m / scale, so fma(s, scale, bias) is score - m and a step
 // without a new maximum has no rescale and no lane exchange. Row sums come from a
 // product with ones. The largest weight is exactly 1 and so has no rounding to
-// bf16: letting scores pass m by up to 2^8 saved the rescales (pair tensor, 60
-// positions 35.8 -> 32.3 us the call) but put the error against float64 at 2.2e-3
-// instead of 2.07e-3 (bf16 operands; the whole-sequence kernel: 2.07e-3).
+// bf16: letting scores pass m by up to 2^8 saved the rescales (a tenth of a pair
+// call at 60 positions) but put the error against float64 at 2.2e-3 instead of
+// 2.07e-3 (bf16 operands; the whole-sequence kernel: 2.07e-3). FINE: a weight is
+// two bf16 numbers, its high and low part, and multiplies V as two products.
 //
 // Biases, fp32 tables in LDS. LINEAR: the offsets the live cells span, laid out
 // (2 dq_max + 1) x (2 dr_max + 1) without clamping while they fit MAX_OFFSETS
@@ -34,13 +35,15 @@
 // 4.8); PAIR: table rows from the pair tensor. Key blocks that hold token or
 // dead keys, and waves whose queries hold tokens, select per lane.
 //
-// Bound: VALU issue (about 45 instructions per 16 x 32 scores: an address, an
-// fma, an exp, half a maximum and half a pack per score) plus the MFMAs, 66 % of
-// the SIMD cycles together, the rest the chain of one chunk. Measured on MI355X:
-// 111 positions, S = 584, H = 3, D = 64 1873 us (one query row per thread) -> 93 us;
-// 150 positions, S = 328, H = 4, D = 32 67 -> 46 us; the pair tensor at 60
-// positions, S = 341, H = 3, D = 64 94 -> 28 us. Two 32-key steps per chunk as a
-// rolled loop keep 139 VGPRs (unrolled 168 with 49 spilled).
+// Bound: no single unit. Counters, 111 positions, S = 584, H = 3, D = 64, FINE: VALU
+// issue 0.50 of the launch's cycles, MFMA 0.18, LDS 0.20; 150 positions, S = 328,
+// H = 4, D = 32 0.45, 0.07 and 0.21: the VALU of a score (an address, an fma, an exp,
+// half a maximum and half a pack) with two to three waves per SIMD that wait 0.4 to
+// 0.5 of their time, in the chain of one chunk. Measured on MI355X: the first
+// shape 1873 us (one query row per thread) -> 106 us (94 with one bf16 per weight),
+// the second 67 -> 47 us; the pair tensor at 60 positions, S = 341, H = 3, D = 64
+// 94 -> 25 us. Two 32-key steps per chunk as a rolled loop keep 145 VGPRs (unrolled
+// 168 with 49 spilled).
 #include <type_traits>
 
 #include "capi.hpp"
@@ -74,8 +77,8 @@ SHRIMP_DEV int clampi(int x, int m) { return min(max(x, -m), m); }
 // LDS byte addresses as plain integers: no base pointer added per read, and
 // the compiler, which takes a read through a pointer into the workgroup's LDS
 // to alias the chunk DMA in flight and waits for it (vmcnt 0), leaves the
-// ordering to the wait and barrier that end each chunk (82.8 -> 81.2 us at
-// D = 64, S = 584, 13.2 -> 12.8 us for a dozen positions at D = 32).
+// ordering to the wait and barrier that end each chunk (2 % at D = 64, S = 584, 3 %
+// for a dozen positions at D = 32).
 SHRIMP_DEV int lds_addr(const void* p) { return (int)(uintptr_t)(lds_cu8*)p; }
 SHRIMP_DEV unsigned lds_u32(int addr) {
   return *(__attribute__((address_space(3))) const unsigned*)(uintptr_t)(unsigned)addr;

@@ -6,7 +6,9 @@
 //   mlp:  s1 = seq + g_attn m (att Wo^T + bo); h = GELU(LN2(s1) W1^T + b1);
 //         seq = s1 + g_mlp m (h W2^T + b2), s1 in fp32, token low parts as mlp.hip
 // with the same folded, packed weights and the same product orientation and
-// fragment orders as qkv.hip and mlp.hip.
+// fragment orders as qkv.hip and mlp.hip. As exact as the linear_kernel sequence
+// before them: two-pass variances and gelu_fine (4 us of the 192-channel MLP
+// together, 2 of the 96-channel one).
 //
 // One workgroup: four waves, MB blocks of 16 rows each, whose activations stay
 // in registers from the first load to the last store. The weights pass through
@@ -19,11 +21,13 @@
 //
 // They replace linear_kernel (two output blocks per pass over the rows, the
 // LayerNorm redone by each of 18 column groups, the hidden rows through HBM) in
-// the attention block. 192 channels, 64 824 rows: qkv 122.8 -> 31.7 us (100 MB,
-// 3.2 TB/s), out_proj + fc1 + fc2 152.8 -> 49.8 us (24 GFLOP, 480 TFLOP/s). 96
-// channels, 49 200 rows: qkv with the zeroed pads 41.3 -> 19.7 us, MLP 58.9 ->
-// 17.6 us. Bound: qkv by HBM and its 8-byte stores, the MLP by MFMA and GELU
-// issue at two waves per SIMD.
+// the attention block. 192 channels, 64 824 rows: qkv 122.8 -> 31.9 us (102 MB,
+// 3.2 TB/s), out_proj + fc1 + fc2 152.8 -> 53.0 us (24 GFLOP, 450 TFLOP/s). 96
+// channels, 49 200 rows: qkv with the zeroed pads 41.3 -> 19.4 us, MLP 58.9 ->
+// 19.4 us. Bound: latency, no unit is at its limit (a copy reaches 5.2 TB/s;
+// counters at 192 channels: qkv VALU 0.18 and MFMA 0.16 of the launch's cycles, MLP
+// 0.32 and 0.18): one and a half waves per SIMD over the launch, in one chain each
+// of rows, stages behind a barrier, and 8-byte stores.
 #include <algorithm>
 
 #include "capi.hpp"

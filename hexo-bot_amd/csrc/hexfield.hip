@@ -33,7 +33,7 @@ using namespace shrimp;
 constexpr int RAY_SLOT_COUNT = 32;
 constexpr int RAY_STEPS = 5;
 constexpr int RA_THREADS = 256;
-constexpr uint32_t RA_STAGE_MAX_LDS = 64 * 1024;
+constexpr uint32_t RA_STAGE_MAX_ROWS = 64 * 1024;  // bytes of the four regions' N rows that are staged
 constexpr uint32_t RA_BIAS_LDS = 96;  // the head pair's 22 fp32 slot biases, padded
 constexpr float LOG2E_F = 1.4426950408889634f;
 
@@ -103,7 +103,8 @@ typedef __attribute__((address_space(3))) void ra_lds_t;
 constexpr uint32_t RA_ABSENT = 0x80000000u;  // past the 2 GiB row resources: zeros
 
 // One of the four staged regions (K and V of two heads): N rows and a zero row,
-// whole 1 KiB DMAs.
+// whole 1 KiB DMAs (at most 17 KiB, 68 KiB and the biases per workgroup, which
+// leaves two per compute unit as 64 KiB would).
 __host__ __device__ constexpr uint32_t ra_region_bytes(int N, int D) {
   return ((uint32_t)(N + 1) * (uint32_t)D * 2 + 1023) / 1024 * 1024;
 }
@@ -120,7 +121,8 @@ __host__ __device__ constexpr uint32_t ra_region_bytes(int N, int D) {
 // out) and LDS holds four per compute unit at N = 256, D = 16. So the row's index
 // slots, reach and queries are requested before the keys are staged, the staging
 // is one round trip, and the eleven gathers carry no branches. B = 700, N = 256,
-// H = 6, D = 16 (136 MB): 60.4 -> 45.2 us, 3.0 TB/s.
+// H = 6, D = 16 (136 MB): 60.4 -> 45.2 us, 3.0 TB/s (VALU 0.33, LDS 0.19 of the
+// launch's cycles; the staged kernel at D = 16 spills 42 SGPRs to VGPR lanes).
 template <int D, bool STAGE>
 __global__ __launch_bounds__(RA_THREADS) void ray_attn_kernel(const shrimp_ray_attn_args a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -768,7 +770,7 @@ extern "C" int shrimp_ray_attn(const shrimp_ray_attn_args* a, void* stream) {
     SHRIMP_REQUIRE(rsn[i] >= a->D && ((int64_t)a->N * rsn[i] + rsh[i]) * 2 < (1LL << 31),
                    "ray_attn: a head pair's rows of a position must span less than 2 GiB");
   SHRIMP_REQUIRE((int64_t)a->B * ((a->H + 1) / 2) < (1LL << 31), "ray_attn: grid too large");
-  const bool stage = g_ray_variant == 0 && 8u * (uint64_t)a->N * a->D <= RA_STAGE_MAX_LDS;
+  const bool stage = g_ray_variant == 0 && 8u * (uint64_t)a->N * a->D <= RA_STAGE_MAX_ROWS;
   hipStream_t s = as_stream(stream);
   switch (a->D) {
     case 16: return launch_ray_attn<16>(*a, stage, s);

@@ -50,8 +50,9 @@ const char* shrimp_last_error(void);
 int shrimp_abi_version(void);
 
 /* Tuning / test switches (no counterpart in the reference).
- * shrimp_conv_variant: 0 = automatic conv kernel choice (a position's rows
- * staged in LDS when they fit, 128x128 tiles per wave for the 128-channel
+ * shrimp_conv_variant: 0 = automatic conv kernel choice (weights streamed
+ * through LDS for the 7-tap conv to 96 and 192 channels from as many or 32; else a
+ * position's rows staged in LDS when they fit, 128x128 tiles per wave for the 128-channel
  * 7-tap conv, and for batches of at most half the compute-unit count one
  * 64-row tile per workgroup so a position's rows spread over several; that
  * split repeats the big-tile kernel's arithmetic where the big-tile kernel

@@ -1303,9 +1303,9 @@ int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_byte
 // table that the whole-sequence kernel builds once for two heads, unless there are
 // enough heads to fill the device and sequences short enough for several
 // whole-sequence workgroups per compute unit. Streamed against whole-sequence, us:
-// H = 4, D = 32 B = 200, S = 136 25.6 / 18.6; B = 384, S = 200 52.5 / 47.3, S = 264
-// 84.0 / 70.4, S = 328 100.6 / 118.3; H = 3, D = 64 B = 400, S = 136 50 / 41, S = 176
-// 54 / 65. To 128 rows and from 1024 heads the streamed one again (B = 800, H = 4,
+// H = 4, D = 32 B = 200, S = 136 27.0 / 19.6; B = 384, S = 200 52.5 / 47.3, S = 264
+// 84.0 / 70.4, S = 328 100.6 / 118.3; H = 3, D = 64 B = 400, S = 136 51.7 / 42.9, S = 176
+// 55.6 / 67.0. To 128 rows and from 1024 heads the streamed one again (B = 800, H = 4,
 // D = 32, S = 72 0.88 times, S = 128 0.86). Below 384 heads it is within 9 % or faster.
 static bool attn_stream_faster(const shrimp_attn_args* a) {
   const int64_t heads = (int64_t)a->B * a->H;

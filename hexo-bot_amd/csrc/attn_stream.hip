@@ -686,7 +686,7 @@ static int launch_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_by
 // 1.27 times the time, 328 rows 1.32, 64 rows (half of a 128-query tile empty) 0.88.
 // The pair form, whose scores wait for their pair rows, takes 32 only where one tile
 // of 128 stands for two of 64 (72 rows, 512 positions, H = 4, D = 32 26.7 us with 16,
-// 22.6 with 32; from 104 rows 0.71 to 1.02 times the time with 16). fine: weights as
+// 22.6 with 32; from 104 rows 0.71 to 1.03 times the time with 16). fine: weights as
 // two bf16 numbers, their product with V as two (dispatch_attn says where; a pair
 // call of at most 256 rows always).
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,

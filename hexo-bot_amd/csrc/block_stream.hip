@@ -7,8 +7,8 @@
 //         seq = s1 + g_mlp m (h W2^T + b2), s1 in fp32, token low parts as mlp.hip
 // with the same folded, packed weights and the same product orientation and
 // fragment orders as qkv.hip and mlp.hip. As exact as the linear_kernel sequence
-// before them: two-pass variances and gelu_fine (4 us of the 192-channel MLP
-// together, 2 of the 96-channel one).
+// before them: two-pass variances and gelu_fine (3 us of the 192-channel MLP
+// together, 1.5 of the 96-channel one).
 //
 // One workgroup: four waves, MB blocks of 16 rows each, whose activations stay
 // in registers from the first load to the last store. The weights pass through

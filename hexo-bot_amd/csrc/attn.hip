@@ -1298,26 +1298,26 @@ bool attn_stream_ok(const shrimp_attn_args* a, int npos);
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
                        uint32_t o_bytes, bool fine, hipStream_t st);
 
-// Where the streamed kernel is the faster one at head dims 32 and 64: the pair form
-// everywhere; the coords form, whose workgroups each build the key codes and the bias
-// table that the whole-sequence kernel builds once for two heads, unless there are
-// enough heads to fill the device and sequences short enough for several
-// whole-sequence workgroups per compute unit. Streamed against whole-sequence, us:
-// H = 4, D = 32 B = 200, S = 136 27.0 / 19.6; B = 384, S = 200 52.5 / 47.3, S = 264
-// 84.0 / 70.4, S = 328 100.6 / 118.3; H = 3, D = 64 B = 400, S = 136 51.7 / 42.9, S = 176
-// 55.6 / 67.0. To 128 rows and from 1024 heads the streamed one again (B = 800, H = 4,
-// D = 32, S = 72 0.88 times, S = 128 0.86). Below 384 heads it is within 9 % or faster.
-static bool attn_stream_faster(const shrimp_attn_args* a) {
-  const int64_t heads = (int64_t)a->B * a->H;
-  if (a->pair != nullptr || 2 * heads < 3 * cu_count()) return true;
-  return a->S <= 128 ? heads >= 4 * cu_count() : a->S > 10240 / a->dpad;
+// Where the streamed kernel takes a call at head dims 32 and 64: by the form and the
+// sequence alone, since its bits are not the whole-sequence kernel's and a position's
+// must not depend on the batch. The pair form always; the coords form, whose workgroups
+// each build the key codes and the bias table that the whole-sequence kernel builds
+// once for two heads, except from 129 rows to where that kernel fits fewer than three
+// workgroups per compute unit. Streamed / whole-sequence, us, by positions:
+//   H = 4, D = 32  S = 72   200 12.8 / 12.5, 800 36.2 / 41.5
+//                  S = 136  1 8.6 / 12.0, 200 27.0 / 19.6, 800 82.1 / 66.1
+//                  S = 264  1 11.5 / 13.6, 400 87.4 / 87.3, 768 155.4 / 132.5
+//                  S = 328  200 55.6 / 73.5, 800 184 / 232
+//   H = 3, D = 64  S = 136  1 9.9 / 12.8, 400 51.7 / 42.9;  S = 176  400 55.6 / 67.0
+static bool attn_stream_takes(const shrimp_attn_args* a) {
+  return a->pair != nullptr || a->S <= 128 || a->S > 10240 / a->dpad;
 }
 
 template <bool PAIR>
 static int dispatch_attn(const shrimp_attn_args* a, float qk_scale, uint32_t qkv_bytes, int npos,
                          int tab_rows, hipStream_t st) {
   if (g_attn_variant == 3) return attn_rows_bf16(a, st);
-  if (g_attn_variant == 0 && attn_stream_ok(a, npos) && attn_stream_faster(a)) {
+  if (g_attn_variant == 0 && attn_stream_ok(a, npos) && attn_stream_takes(a)) {
     // Weights as two bf16 numbers where one would be less exact than the kernel that
     // stood here (relative error against float64, of which the output's own rounding
     // is 1.66e-3): past the whole-sequence kernels' sequences, where the chunked kernel

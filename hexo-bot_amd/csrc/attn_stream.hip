@@ -42,8 +42,9 @@
 // 0.5 of their time, in the chain of one chunk. Measured on MI355X: the first
 // shape 1873 us (one query row per thread) -> 106 us (94 with one bf16 per weight),
 // the second 67 -> 47 us; the pair tensor at 60 positions, S = 341, H = 3, D = 64
-// 94 -> 25 us. Two 32-key steps per chunk as a rolled loop keep 145 VGPRs (unrolled
-// 168 with 49 spilled).
+// 94 -> 25 us. Two 32-key steps per chunk as a rolled loop keep 147 VGPRs (unrolled
+// 168 with 49 spilled). A query's bits depend on its own rows only, not on the tiling
+// or on the queries beside it.
 #include <type_traits>
 
 #include "capi.hpp"
@@ -149,19 +150,23 @@ struct StreamLds {      // LDS byte addresses
   int npos;
 };
 
-// Key blocks of a chunk scored together: more keep more independent products
-// in flight, fewer fit the registers of three waves per SIMD.
-template <int D, int QB>
+// Key blocks scored together, around one offset: the same at both tilings of the
+// coords form, so that a query's bits do not depend on the tiling and with it on the
+// batch. Two, which fit the registers of three waves per SIMD at QB = 2 (the 16-query
+// tiling alone would take four: one position at S = 500, D = 32 13.2 against 15.1 us);
+// four for the pair form, which has one tiling.
+template <int PATH>
 constexpr int stream_nkb() {
-  return QB == 2 ? 2 : 4;
+  return PATH == PATH_PAIR ? 4 : 2;
 }
 
 // NKB blocks of 16 keys from key k0, K and V rows at LDS bytes kbuf, vbuf;
 // bit kb of `special` (wave-uniform): block kb selects its biases per lane.
-template <int D, int QB, int PATH, int NKB, bool FINE>
+template <int D, int QB, int PATH, bool FINE>
 SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, const StreamLds& s,
                              int k0, int L, int special, int kbuf, int vbuf, int lr, int lg,
-                             float scale, const unsigned (&pd)[QB][NKB]) {
+                             float scale, const unsigned (&pd)[QB][stream_nkb<PATH>()]) {
+  constexpr int NKB = stream_nkb<PATH>();
   constexpr int KS = D / 32, KD = D / 16, RB = 2 * D;
   f32x4 v[QB][NKB];
   const int ksw = swz<D>(lr);
@@ -250,7 +255,9 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
     }
     return __builtin_amdgcn_ballot_w64(bad) != 0;
   };
-  // moves them; whether one fell far
+  // moves them; whether one fell far. Queries whose offset stays (delta 0) keep their
+  // bits, whatever the others of the wave do.
+  bool drop[QB];
   auto shift = [&]() -> bool {
     bool far = false;
 #pragma unroll
@@ -261,7 +268,8 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
       const float delta = seen ? fmaxf(g, 0.f) : (g > 0.1f * AST_NEG_BIG ? g : 0.f);
       const float alpha = seen ? __builtin_amdgcn_exp2f(-delta) : 0.f;
       w.m[qb] += delta;
-      far |= m0 > FAR_OFFSET && m0 > 2.f * fabsf(w.m[qb]);
+      drop[qb] = m0 > FAR_OFFSET && m0 > 2.f * fabsf(w.m[qb]);
+      far |= drop[qb];
       const float c = -w.m[qb] * s.inv_scale, lsum = w.l[qb][0] * alpha;
       w.cinit[qb] = f32x4{c, c, c, c};
       w.l[qb] = f32x4{lsum, lsum, lsum, lsum};
@@ -283,7 +291,16 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
     // again around the new one.
 #pragma unroll 1
     for (int n = 0; __builtin_expect(far, 0) && n < MAX_RESCORES; ++n) {
+      f32x4 keep[QB][NKB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) keep[qb][kb] = v[qb][kb];
       score();
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) v[qb][kb] = drop[qb] ? v[qb][kb] : keep[qb][kb];
       (void)over();
       far = shift();
     }
@@ -615,7 +632,6 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
       }
       if (active) {
         const int kbuf = lds0 + buf * 2 * CB, vbuf = kbuf + CB;
-        constexpr int NKB = stream_nkb<D, QB>();
         int special;
         if constexpr (PAIR) {
           const int over = L - c * KC;  // keys of the chunk inside the bound
@@ -623,6 +639,7 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
         } else {
           special = tok ? 15 : __builtin_amdgcn_readfirstlane((int)lds_u8(lds_addr(flags) + c));
         }
+        constexpr int NKB = stream_nkb<decltype(path)::value>();
 #pragma unroll 1
         for (int kb = 0; kb < 4 && c * KC + kb * 16 < L; kb += NKB) {
           unsigned p[QB][NKB];
@@ -630,9 +647,9 @@ __global__ __launch_bounds__(256, QB == 2 ? 3 : 4) void attn_stream_kernel(const
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-              for (int i = 0; i < NKB; ++i) p[qb][i] = kb == 0 ? pd[qb][i] : pd[qb][(4 - NKB) + i];
+              for (int i = 0; i < NKB; ++i) p[qb][i] = pd[qb][i];
           }
-          stream_chunk<D, QB, decltype(path)::value, NKB, FINE>(
+          stream_chunk<D, QB, decltype(path)::value, FINE>(
               a, w, s, c * KC + kb * 16, L, special >> kb, kbuf + kb * 16 * RB, vbuf + kb * 16 * RB,
               lr, lg, scale, p);
           __builtin_amdgcn_sched_barrier(0);
@@ -680,33 +697,28 @@ static int launch_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_by
   return check_launch("attn");
 }
 
-// 32 queries per wave (each K and V fragment read feeds two products) for a coords
-// call of more than 64 rows once such tiles give every compute unit two workgroups,
-// else 16. Measured, 16 against 32: coords at 768 positions, H = 4, D = 32 200 rows
-// 1.27 times the time, 328 rows 1.32, 64 rows (half of a 128-query tile empty) 0.88.
-// The pair form, whose scores wait for their pair rows, takes 32 only where one tile
-// of 128 stands for two of 64 (72 rows, 512 positions, H = 4, D = 32 26.7 us with 16,
-// 22.6 with 32; from 104 rows 0.71 to 1.03 times the time with 16). fine: weights as
-// two bf16 numbers, their product with V as two (dispatch_attn says where; a pair
-// call of at most 256 rows always).
+// Coords: 32 queries per wave (each K and V fragment read feeds two products) past 64
+// rows once such tiles give every compute unit two workgroups, else 16, with the same
+// bits. Measured at 768 positions, H = 4, D = 32, 16 against 32: 200 rows 1.27 times the
+// time, 328 rows 1.32, 64 rows (half of a 128-query tile empty) 0.88. Pair: 16, whose
+// scores wait for their pair rows (32 against them from 104 rows 0.97 to 1.41 times the
+// time; at 72 rows, 512 positions, H = 4, D = 32 22.6 us for 26.7, left for one set of
+// bits at every batch). fine: weights as two bf16 numbers, their product with V as
+// two (dispatch_attn says where).
 int launch_attn_stream(const shrimp_attn_args* a, float scale, uint32_t qkv_bytes, int npos,
                        uint32_t o_bytes, bool fine, hipStream_t st) {
-  const bool pair = a->pair != nullptr;
-  const bool wide = a->S > 64 && (!pair || a->S <= 96) &&
-                    (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
+  const bool wide = a->S > 64 && (int64_t)a->B * a->H * ((a->S + 127) / 128) >= 2 * cu_count();
 #define AST_LAUNCH(...)                                                                       \
   do {                                                                                        \
     if (fine) return launch_stream<__VA_ARGS__, true>(a, scale, qkv_bytes, npos, o_bytes, st); \
     return launch_stream<__VA_ARGS__, false>(a, scale, qkv_bytes, npos, o_bytes, st);         \
   } while (0)
   if (a->dpad == 64) {
-    if (pair && wide) return launch_stream<64, 2, true, true>(a, scale, qkv_bytes, npos, o_bytes, st);
-    if (pair) AST_LAUNCH(64, 1, true);
+    if (a->pair != nullptr) AST_LAUNCH(64, 1, true);
     if (wide) AST_LAUNCH(64, 2, false);
     AST_LAUNCH(64, 1, false);
   }
-  if (pair && wide) return launch_stream<32, 2, true, true>(a, scale, qkv_bytes, npos, o_bytes, st);
-  if (pair) AST_LAUNCH(32, 1, true);
+  if (a->pair != nullptr) AST_LAUNCH(32, 1, true);
   if (wide) AST_LAUNCH(32, 2, false);
   AST_LAUNCH(32, 1, false);
 #undef AST_LAUNCH

@@ -61,8 +61,9 @@ int shrimp_abi_version(void);
  * 3 = as 0 without the small-batch row split; other values only query.
  * Returns the previous setting. Process-wide.
  * shrimp_attn_variant: 0 = automatic (padded head dims 32 and 64: keys streamed
- * through LDS 64 at a time, where that is faster and the q / k / v rows lie on
- * 16-byte boundaries, lut_m <= 28 and the tables fit the LDS; else two heads per attention workgroup
+ * through LDS 64 at a time, for the pair form and for coords of up to 128 rows or more
+ * than 10240 / dpad, where the q / k / v rows lie on 16-byte boundaries, lut_m <= 28
+ * and the tables fit the LDS; else two heads per attention workgroup
  * when their K/V fit the 64 KiB budget, on eight waves at padded head dim 16, else
  * four; one head per workgroup with up to the device's per-workgroup LDS for
  * longer sequences; beyond that the chunked kernel of shrimp_attn_f32 on bf16

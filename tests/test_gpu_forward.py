@@ -403,6 +403,23 @@ def test_batches_above_the_limit_split_bit_exact(cfg4_batch):
         assert torch.equal(split[key], full[key]), key
 
 
+@pytest.mark.parametrize("channels,heads", [(96, 4), (192, 3)])
+def test_weight_streamed_widths_same_bits_at_any_batch(channels, heads):
+    """96 and 192 channels: a position's outputs are the same bits alone, among
+    eight and in a batch on the other side of every kernel's row-tiling rule."""
+
+    from shrimp import synthetic
+
+    b = synthetic.position_batch("cfg4", 160)
+    net = _net(channels, heads, "CCA", seed=5)
+    args = [torch.as_tensor(b[k]).to(DEV) for k in ("feats", "nbr", "mask", "coords")]
+    full = net.forward_policy_value(*args, request_moves_left=True)
+    for lo, hi in ((0, 1), (40, 48), (80, 160)):
+        part = net.forward_policy_value(*(t[lo:hi] for t in args), request_moves_left=True)
+        for key in ("policy", "value", "moves_left"):
+            assert torch.equal(part[key], full[key][lo:hi]), (key, lo, hi)
+
+
 @pytest.mark.parametrize("graphs", [False, True], ids=["eager", "graphs"])
 def test_evaluator_matches_reference_reply(golden, graphs):
     """The reference evaluator's reply (ShrimpEvaluator(net, "cpu"), written

@@ -1268,9 +1268,8 @@ def _coords_attention_ref(q, k, v, coords, mask, lens, table, nt):
 
 # head dims 32 and 64 stream the keys through LDS 64 at a time: sequence
 # lengths around a chunk and around the two query tilings (64 queries per
-# workgroup, or 128 past 64 rows once B H tiles reach two per compute unit; at most
-# 320 rows at head dim 32 and 160 at 64 that is from 1024 heads, the whole-sequence
-# kernels taking 384 to 1024),
+# workgroup, or 128 past 64 rows once B H tiles reach two per compute unit; from 129
+# to 320 rows at head dim 32 and 160 at 64 the whole-sequence kernels),
 # spans on either side of the unclamped table (window 20: linear, 60: clamped),
 # lengths of 0, inside the tokens and ragged, dead cells whose K and V rows hold
 # NaN, a head dim below its padding, an odd head count
@@ -1316,6 +1315,51 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     assert torch.isfinite(got).all()
     # p and the result are rounded to bf16 (2^-9 each) around |v| up to 4.5
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
+
+
+# A position's bits are those of any batch: one position, eight and the whole batch,
+# which differ in the streamed kernel's query tiling or stand on either side of the
+# whole-sequence kernels' splits. Scores spread by a gain, and a table whose first
+# key block sets offsets that later ones leave far behind (scores formed again).
+@pytest.mark.parametrize("gain,low", [(1.0, False), (20.0, False), (1.0, True)])
+@pytest.mark.parametrize("H,S,d", [(4, 72, 24), (3, 72, 64), (4, 136, 32), (3, 136, 64), (4, 264, 24),
+                                   (3, 264, 64), (4, 330, 32), (3, 584, 64)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_attn_bits_at_any_batch(H, S, d, gain, low, pair):
+    from shrimp import ops
+    from shrimp.geometry import CELL_LUT_M, cell_bias_lut
+
+    g = torch.Generator().manual_seed(S + d)
+    B, dp = 200 if S < 300 else 96, max(16, -(-d // 16) * 16)
+    q, k, v = (torch.randn(B, H, S, d, generator=g) for _ in range(3))
+    table = torch.randn(237, H, generator=g)
+    lens = torch.randint(S // 2, S + 1, (B,), generator=g).to(torch.int32)
+    if low:  # the first 70 keys far below the rest, for every other query
+        table[:1 if pair else 200] = -1e9
+    rows = torch.randint(1, 237, (B, S, S), generator=g, dtype=torch.uint8) if pair else None
+    if pair:
+        rows[:, ::2, :70] = 0
+    at = torch.stack([torch.randperm(676, generator=g)[:S] for _ in range(B)])
+    coords = torch.stack([at // 26, at % 26], -1).to(torch.int32)
+    btab, xtab = ops.attn_bias_table(table.to(DEV), torch.from_numpy(cell_bias_lut()).to(DEV))
+    pad = lambda t: torch.nn.functional.pad(t, (0, dp - d)).to(DEV, torch.bfloat16).contiguous()
+    qd, kd, vd = pad(q * gain), pad(k), pad(v)
+    ld, cd, md = lens.to(DEV), coords.to(DEV), torch.ones(B, S, dtype=torch.uint8, device=DEV)
+    rd, td = rows.to(DEV) if pair else None, table.to(DEV)
+
+    def run(lo, hi):
+        n, out = hi - lo, torch.empty(hi - lo, H, S, d, dtype=torch.bfloat16, device=DEV)
+        kw = dict(pair=rd[lo:hi], p_sb=S * S, p_sq=S, table2=td) if pair else dict(
+            coords=cd[lo:hi], mask8=md[lo:hi], btab=btab, xtab=xtab, lut_m=CELL_LUT_M)
+        ops.launch_attn(q=qd[lo:hi], k=kd[lo:hi], v=vd[lo:hi], qkv_sb=H * S * dp, qkv_sh=S * dp,
+                        seq_lens=ld[lo:hi], o=out, o_sb=H * S * d, o_sh=S * d, o_sr=d, B=n, S=S, H=H,
+                        d=d, dpad=dp, n_tokens=0, **kw)
+        return out
+
+    full = run(0, B)
+    assert torch.isfinite(full.float()).all()
+    for lo, hi in ((0, 1), (3, 11), (B - 1, B), (0, B // 2)):
+        assert torch.equal(run(lo, hi), full[lo:hi]), (lo, hi)
 
 
 # The longest sequences that the streamed kernel's key tables fit beside its chunks
@@ -1379,8 +1423,7 @@ def test_attn_streamed_fallback(d, how):
     close(out, want, atol=1e-2, what=f"d={d} {how}")
 
 
-# The pair form on both query tilings (128 queries per workgroup from 65 to 96 rows
-# once those are two per compute unit: B = 172, H = 3) at sequence lengths around the pair loader's four keys, a 16-key block, a
+# The pair form on few and many workgroups at sequence lengths around the pair loader's four keys, a 16-key block, a
 # chunk and a wave's queries, to 256 rows with weights of two bf16 numbers and
 # past them of one; ragged bounds, an odd head count. Eight positions compared.
 @pytest.mark.parametrize("B,H", [(3, 3), (172, 3)])

@@ -313,11 +313,22 @@ SHRIMP_DEV void stream_chunk(const shrimp_attn_args& a, StreamQuery<D, QB>& w, c
       float p[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(v[qb][kb][j]);
-      const u32x2 hi{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
-      pf[qb][kb] = hi;
-      if constexpr (FINE)
-        pl[qb][kb] = u32x2{pack_bf16x2(p[0] - bf16_lo(hi.x), p[1] - bf16_hi(hi.x)),
-                           pack_bf16x2(p[2] - bf16_lo(hi.y), p[3] - bf16_hi(hi.y))};
+      if constexpr (FINE) {
+        // high part cut, not rounded, and below the weight: the low part is positive,
+        // so an infinite value of V stays one (0 or less times it would be a NaN)
+        unsigned t[4];
+        float r[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          t[j] = __float_as_uint(p[j] * (1.f - 0x1p-16f));
+          r[j] = p[j] - __uint_as_float(t[j] & 0xFFFF0000u);
+        }
+        pf[qb][kb] = u32x2{__builtin_amdgcn_perm(t[1], t[0], 0x07060302u),
+                           __builtin_amdgcn_perm(t[3], t[2], 0x07060302u)};
+        pl[qb][kb] = u32x2{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
+      } else {
+        pf[qb][kb] = u32x2{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])};
+      }
     }
   __builtin_amdgcn_sched_barrier(0);
   const unsigned one2 = 0x3F803F80u;

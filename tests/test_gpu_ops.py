@@ -1317,6 +1317,29 @@ def test_attn_streamed_keys(B, H, S, d, dpad, nt, window, gain):
     close(got[rows], want[rows], atol=2e-2, rtol=1e-2, what="streamed attention")
 
 
+# An infinite value gives an infinity wherever a key that holds one has weight, with
+# weights of two bf16 numbers (40 and, past the whole-sequence kernels, 700 rows) as
+# of one (300); a NaN key, query or value a NaN; other positions stay finite.
+@pytest.mark.parametrize("S", [40, 300, 700])
+@pytest.mark.parametrize("d", [16, 32, 64])
+def test_attn_pair_special_values(d, S):
+    g = torch.Generator().manual_seed(S + d)
+    B, H = 4, 2
+    q, k, v = (bf(torch.randn(B, H, S, d, generator=g)) for _ in range(3))
+    v[0, 0, 5, 3], v[0, 1, S - 1, 0] = float("inf"), -float("inf")
+    v[1, 0, 7, 1] = k[2, 1, 2, 2] = q[2, 0, 9, 0] = float("nan")
+    pair = torch.zeros(B, S, S, dtype=torch.uint8)
+    table2, lens = torch.zeros(2, H), torch.full((B,), S, dtype=torch.int32)
+    dev = lambda t: t.to(DEV, torch.bfloat16)
+    got = torch.ops.shrimp.attn_pair(dev(q), dev(k), dev(v), pair.to(DEV), table2.to(DEV), lens.to(DEV))
+    want = ofwd.attn_pair(q, k, v, pair, table2.double(), lens)
+    got = got.cpu().double()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+    fin = want.isfinite()
+    close(got[fin], want[fin], atol=1e-2, what=f"d={d} S={S}")
+
+
 # A position's bits are those of any batch: one position, eight and the whole batch,
 # which differ in the streamed kernel's query tiling or stand on either side of the
 # whole-sequence kernels' splits. Scores spread by a gain, and a table whose first
